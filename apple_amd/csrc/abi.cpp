@@ -444,25 +444,24 @@ int elem_eval_impl(apl_mesh* m, int material, const void* mu, const void* lam, c
         if (egh & b) passes[np++] = b;
     for (int i = 0; i < np; ++i) {
       const unsigned pw = passes[i];
-      if (launch_elem(m, material, pw, mu, lam, u, nullptr, nullptr, nullptr, grad, hess_diag, acc, 0, s, 0, nullptr,
-                      ws))
+      if (launch_elem(m, material, pw, mu, lam, u, nullptr, grad, hess_diag, acc, s, nullptr, ws))
         return -1;
       if (launch_finish(m, pw, grad, hess_diag, (pw & W_E) ? energy : nullptr, nullptr, acc, nullptr, s, ws))
         return -1;
     }
   }
   if (w & W_HP) {
-    if (launch_elem(m, material, W_HP, mu, lam, u, p, nullptr, nullptr, hess_prod, nullptr, acc, 0, s, 0, nullptr, ws))
+    if (launch_elem(m, material, W_HP, mu, lam, u, p, hess_prod, nullptr, acc, s, nullptr, ws))
       return -1;
     if (launch_finish(m, W_HP, hess_prod, nullptr, nullptr, nullptr, acc, nullptr, s, ws)) return -1;
   }
   if (w & W_HQ) {
-    if (launch_elem(m, material, W_HQ, mu, lam, u, p, nullptr, nullptr, nullptr, nullptr, acc, 0, s, 0, nullptr, ws))
+    if (launch_elem(m, material, W_HQ, mu, lam, u, p, nullptr, nullptr, acc, s, nullptr, ws))
       return -1;
     if (launch_finish(m, W_HQ, nullptr, nullptr, nullptr, hess_quad, acc, nullptr, s, ws)) return -1;
   }
   if (w & W_MIX) {
-    if (launch_elem(m, material, W_MIX, mu, lam, u, p, nullptr, nullptr, dmu, dlam, acc, 0, s, 0, nullptr, ws))
+    if (launch_elem(m, material, W_MIX, mu, lam, u, p, dmu, dlam, acc, s, nullptr, ws))
       return -1;
   }
   return 0;
@@ -504,8 +503,8 @@ int apl_elem_mixed_activation(apl_mesh* m, const void* mu, const void* lam, cons
   (void)hipGetLastError();  // drop errors left by unrelated earlier HIP calls
   const unsigned w = dmu != nullptr ? (W_MIX | W_MIXA) : W_MIXA;
   // a model mesh: dact of its muscle-law tets, dmu / dlam of every tet
-  return launch_elem(m, m->model ? MAT_MODEL : MAT_MUSCLE, w, mu, lam, u, p, nullptr, nullptr, dmu, dlam,
-                     accumulate ? 1 : 0, 0, (hipStream_t)stream, 0, dact);
+  return launch_elem(m, m->model ? MAT_MODEL : MAT_MUSCLE, w, mu, lam, u, p, dmu, dlam,
+                     accumulate ? 1 : 0, (hipStream_t)stream, dact);
 }
 
 }  // extern "C"
@@ -577,13 +576,13 @@ int apl_bench_elem_pass(apl_mesh* m, int material, unsigned what, const void* mu
   if (ms_kernel != nullptr) {
     APL_CHECK_HIP(hipEventRecord(ev[0], s));
     for (int it = 0; it < iters && rc == 0; ++it)
-      rc = launch_elem(m, material, w, mu, lam, u, p, nullptr, nullptr, out_a, out_b, 0, 0, s);
+      rc = launch_elem(m, material, w, mu, lam, u, p, out_a, out_b, 0, s);
     APL_CHECK_HIP(hipEventRecord(ev[1], s));
   }
   if (ms_pass != nullptr && rc == 0) {
     APL_CHECK_HIP(hipEventRecord(ev[2], s));
     for (int it = 0; it < iters && rc == 0; ++it) {
-      rc = launch_elem(m, material, w, mu, lam, u, p, nullptr, nullptr, out_a, out_b, 0, 0, s);
+      rc = launch_elem(m, material, w, mu, lam, u, p, out_a, out_b, 0, s);
       if (rc == 0)
         rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0,
                            nullptr, s);
@@ -634,7 +633,7 @@ int apl_bench_elem_graph(apl_mesh* m, int material, unsigned what, const void* m
     int rc = 0;
     if (hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal) != hipSuccess) rc = -1;
     for (int it = 0; it < iters && rc == 0; ++it) {
-      rc = launch_elem(m, material, w, mu, lam, u, p, nullptr, nullptr, out_a, out_b, 0, 0, cs);
+      rc = launch_elem(m, material, w, mu, lam, u, p, out_a, out_b, 0, cs);
       if (rc == 0)
         rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0,
                            nullptr, cs);

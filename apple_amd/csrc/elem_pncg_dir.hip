@@ -1,0 +1,7 @@
+// The PNCG's step and quadratic-form pass (elem_kernel.h, W_DIR).
+#include "elem_solve_impl.h"
+
+namespace apl {
+APL_SOLVE_PASS(W_HQ | W_DIR, float)
+APL_SOLVE_PASS(W_HQ | W_DIR, double)
+}  // namespace apl

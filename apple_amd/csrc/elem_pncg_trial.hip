@@ -1,0 +1,7 @@
+// The PNCG's trial pass (elem_kernel.h, W_TRIAL).
+#include "elem_solve_impl.h"
+
+namespace apl {
+APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL, float)
+APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL, double)
+}  // namespace apl

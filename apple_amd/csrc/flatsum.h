@@ -44,4 +44,35 @@ __device__ inline void flat_column_sums(const double* __restrict__ p, long long 
   __syncthreads();
 }
 
+// The sum that flat_column_sums<2, NT> gives for the second column of a
+// two-column table, of that column alone (p[0 .. n), contiguous): the same
+// additions in the same order.  There column 1 of row b goes to thread
+// 2 (b mod NT/2) + 1, so here NT/2 threads hold the odd threads' sums and a
+// group of 32 lanes stands for one of its waves.  Valid in every thread.
+template <int NT>
+__device__ inline double flat_sum_odd(const double* __restrict__ p, long long n, double* sm) {
+  constexpr int H = NT / 2;
+  const int t = threadIdx.x;
+  double a[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  if (t < H) {
+    for (long long f = t; f < n; f += 8LL * H) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = f + (long long)u * H < n ? p[f + (long long)u * H] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[u] += v[u];
+    }
+    double s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+#pragma unroll
+    for (int off = 16; off >= 1; off >>= 1) s += __shfl_down(s, off, 32);
+    if ((t & 31) == 0) sm[t >> 5] = s;
+  }
+  __syncthreads();
+  double r = 0.0;
+#pragma unroll
+  for (int i = 0; i < H / 32; ++i) r += sm[i];
+  __syncthreads();
+  return r;
+}
+
 }  // namespace apl

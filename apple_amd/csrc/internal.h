@@ -16,6 +16,7 @@ constexpr int NTH = 256;       // threads per element / vector block
 constexpr int MAX_CH = 6;      // scatter channels per incidence (grad + hdiag)
 constexpr int N_DOTS = 16;     // per vertex-block partial dot products
 constexpr int RED_STRIDE = 2;  // per element block: energy, quadratic form
+constexpr int N_VARIANTS = 13;  // element pass variants (elem_kernel.h, variant_index)
 // material id of a model mesh's launches: every law over its own blocks
 constexpr int MAT_MODEL = 3;
 
@@ -66,7 +67,7 @@ struct apl_mesh {
   apl::Layout L;
   apl::DevLayout d;
   size_t device_bytes = 0;
-  int grid_cache[3][512] = {};  // persistent grid per (material, pass variant, FP64 displacements, filtered)
+  int grid_cache[3][2 * apl::N_VARIANTS] = {};  // persistent grid per (material, pass variant, filtered)
   int refs = 1;                 // the caller's handle plus one per solver built on the mesh
   int grid_pct = 0;             // persistent element grid, percent of occupancy x CUs (autotuned; 0: per-pass default)
   const void* activation = nullptr;  // caller-owned (T, 6) muscle activation, read at every muscle launch
@@ -111,11 +112,9 @@ int elem_eval_impl(apl_mesh* m, int material, const void* mu, const void* lam, c
                    void* dmu, void* dlam, hipStream_t s, const Workspace* ws);
 
 // element pass: per-slot partial sums into the partial workspace (scatter
-// passes), per-block energy/quadratic-form sums, or per-tet outputs (mixed);
-// x_f64: x holds FP64 displacements while the mesh is FP32 (solver passes)
+// passes), per-block energy/quadratic-form sums, or per-tet outputs (mixed)
 int launch_elem(apl_mesh* m, int material, unsigned what, const void* mu, const void* lam,
-                const void* x, const void* p, const double* alpha, const int32_t* active,
-                void* out_a, void* out_b, int accumulate, int grid_override, hipStream_t s, int x_f64 = 0,
+                const void* x, const void* p, void* out_a, void* out_b, int accumulate, hipStream_t s,
                 void* out_c = nullptr, const Workspace* ws = nullptr);
 // vertex sums of the slot partials into the (V,3) outputs
 // Finish pass of an element pass in one launch: vertex sums of the slot
@@ -131,7 +130,7 @@ bool needs_lambda(const apl_mesh* m, int material);
 // largest block window (distinct vertices per block) whose LDS every element
 // pass variant of a mesh of this dtype fits
 int nloc_limit(int dtype);
-int elem_grid(apl_mesh* m, int material, unsigned what, int x_f64 = 0, bool filtered = false);
+int elem_grid(apl_mesh* m, int material, unsigned what);
 // device setup (setup.hip): the element data (inverse rest shapes, dV *
 // fraction) of a created mesh from host cells / points / fraction, and the
 // read-back of the element data in the caller's tet order (T x 9, T)

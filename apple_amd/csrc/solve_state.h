@@ -1,0 +1,160 @@
+// Per-instance state of the device solvers and the scalar decisions taken on
+// it, shared by the solver's scalar kernels and its element passes.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+
+#include "../../include/apple_amd.h"
+#include "internal.h"
+
+namespace apl {
+
+enum : int { D_G2 = 0, D_GPG, D_GPG0, D_GPGC, D_GPGC0, D_GCPGC, D_GCPGC0, D_GTP, D_GCP, D_HSUM, D_HCNT, D_EXT, D_PP, D_E };
+static_assert(D_E < N_DOTS, "dot table too small");
+static_assert(D_PP < N_DOTS, "dot slots");
+
+// One instance's solver state, one record per instance.  `cur` names the
+// buffer of the pair (iterate, direction) that holds the committed point: an
+// accepted step flips it, and the direction pass that follows writes the new
+// point there from the other one, so blocks that share a vertex all read the
+// old values whatever order they run in.
+struct alignas(16) InstState {
+  double f, gd, alpha, alpha_commit, beta, gnorm0, gnorm, pmean, f_first, pHp, gbest, f_mark, f0;
+  int32_t status, act_eval, act_dir, commit, n_steps, n_evals, ls_step, n_backtracks, phase, restarts, best_step,
+      ls_last, cur;
+};
+
+struct Params {
+  double rtol, atol, overstep, c1, wolfe_delta, wolfe_eps, beta_max;
+  int max_steps, max_backtracking, stall_steps;
+};
+
+// per-instance decision from the instance's dot totals
+__device__ inline void pncg_scalar_step(InstState& s, const Params& P, const double* tot) {
+  const double fE = tot[D_E];
+  const double ft = fE + tot[D_EXT];
+  const double gn = sqrt(tot[D_G2]);
+  const int phase = s.phase;
+  s.n_evals += 1;
+  bool accept;
+  if (phase != 1) {
+    accept = true;
+  } else {
+    const double f0 = s.f, a = s.alpha, gd = s.gd;
+    const bool fin = isfinite(ft);
+    const bool armijo = fin && ft <= f0 + P.c1 * a * gd;
+    const bool wolfe = P.wolfe_delta > 0.0 && fin && ft <= f0 + P.wolfe_eps * fabs(f0) &&
+                       tot[D_GTP] <= (2.0 * P.wolfe_delta - 1.0) * gd;
+    accept = armijo || wolfe;
+  }
+  if (accept) {
+    s.alpha_commit = phase == 1 ? s.alpha : 0.0;
+    s.f0 = phase == 0 ? ft : s.f;  // the line search's start and end energies
+    s.ls_last = s.ls_step;
+    s.f = ft;
+    s.gnorm = gn;
+    s.commit = 1;
+    s.cur ^= 1;
+    if (phase == 0) {
+      s.gnorm0 = gn;
+      s.f_first = ft;
+    }
+    if (phase == 1) {
+      s.n_steps += 1;
+      s.restarts = 0;
+    }
+    // progress marker: the last step that lowered the best gradient norm by
+    // 10% or the energy, since the previous marker, by more than the energy
+    // noise the approximate-Wolfe test tolerates (10 wolfe_eps relative)
+    const bool g_prog = gn < 0.9 * s.gbest;
+    const double f_tol = fmax(10.0 * P.wolfe_eps, 1e-12) * fabs(ft);
+    const bool f_prog = !(s.f_mark - ft <= f_tol);
+    if (g_prog) s.gbest = gn;
+    if (g_prog || f_prog) {
+      s.best_step = s.n_steps;
+      s.f_mark = ft;
+    }
+    int status = APL_RUNNING;
+    if (!isfinite(gn) || !isfinite(ft))
+      status = APL_NON_FINITE;
+    else if (gn <= P.rtol * s.gnorm0 || gn <= P.atol)
+      status = APL_PRIMARY_SUCCESS;
+    else if (s.n_steps >= P.max_steps)
+      status = APL_MAX_STEPS_REACHED;
+    else if (P.stall_steps > 0 && s.n_steps - s.best_step >= P.stall_steps && s.gbest <= 1e3 * P.rtol * s.gnorm0)
+      status = APL_STAGNATION;  // within 3 decades of the target: the rounding floor of the gradient
+    s.status = status;
+    if (status == APL_RUNNING) {
+      const double pm = tot[D_HCNT] > 0.0 ? tot[D_HSUM] / tot[D_HCNT] : 1.0;
+      s.pmean = pm;
+      const double gPg = tot[D_GPG] + tot[D_GPG0] / pm;
+      double beta = 0.0;
+      if (phase == 1) {
+        const double gPgc = tot[D_GPGC] + tot[D_GPGC0] / pm;
+        const double gcPgc = tot[D_GCPGC] + tot[D_GCPGC0] / pm;
+        const double yp = tot[D_GTP] - tot[D_GCP];
+        if (fabs(yp) > 1e-300) {
+          const double gPy = gPg - gPgc;
+          const double yPy = gPg - 2.0 * gPgc + gcPgc;
+          beta = gPy / yp - (yPy / yp) * (tot[D_GTP] / yp);
+        } else {
+          beta = INFINITY;
+        }
+        if (!isfinite(beta) || fabs(beta) > P.beta_max) beta = 0.0;
+      }
+      double gd = -gPg + beta * tot[D_GTP];
+      if (!(isfinite(gd) && gd < 0.0)) {
+        beta = 0.0;
+        gd = -gPg;
+      }
+      s.beta = beta;
+      s.gd = gd;
+      s.act_dir = 1;
+    } else {
+      s.act_dir = 0;
+      s.act_eval = 0;
+    }
+    s.ls_step = 0;
+    s.phase = 1;
+  } else {
+    s.commit = 0;
+    s.act_dir = 0;
+    s.ls_step += 1;
+    s.n_backtracks += 1;
+    const double a = s.alpha * 0.5;
+    if (s.ls_step > P.max_backtracking || !(a > 0.0)) {
+      if (s.restarts >= 1) {
+        s.status = APL_STAGNATION;
+        s.act_eval = 0;
+      } else {
+        // restart from x with steepest descent: re-evaluate at alpha = 0
+        s.restarts += 1;
+        s.phase = 2;
+        s.alpha = 0.0;
+        s.ls_step = 0;
+      }
+    } else {
+      s.alpha = a;
+    }
+  }
+}
+
+// step length of a new direction from its quadratic form; the iteration's
+// flags are cleared
+__device__ inline void pncg_alpha_step(InstState& s, const Params& P, double pHp) {
+  if (s.act_dir != 0) {
+    s.pHp = pHp;
+    double a = -s.gd / pHp;
+    if (isnan(a)) a = 0.0;
+    else if (a == -INFINITY) a = 0.0;
+    else if (a == INFINITY) a = 1.0;
+    if (!(a > 0.0 && isfinite(a))) a = 1.0;
+    s.alpha = a * P.overstep;
+  }
+  s.commit = 0;
+  s.act_dir = 0;
+}
+
+}  // namespace apl
