@@ -36,13 +36,12 @@ struct FinishArgs {
 
 template <class R, int NCH>
 __global__ __launch_bounds__(NTH) void finish_kernel(FinishArgs<R> A) {
-  __shared__ double red[2 * (NTH / 64 + 1)];
+  __shared__ double eq[2 * (NTH / 64 + 1)];
   if ((int)blockIdx.x < A.ninst) {
     const int i = (int)blockIdx.x;
     if (A.active != nullptr && A.active[i] == 0) return;
     const long long b0 = A.inst_blk_off[i];
-    double eq[2];
-    flat_column_sums<2, NTH>(A.blk_red + RED_STRIDE * b0, RED_STRIDE * (A.inst_blk_off[i + 1] - b0), red, eq);
+    flat_column_sums<2, NTH>(A.blk_red + RED_STRIDE * b0, RED_STRIDE * (A.inst_blk_off[i + 1] - b0), eq);
     if (threadIdx.x == 0) {
       if (A.out_e != nullptr) A.out_e[i] = A.accumulate ? A.out_e[i] + eq[0] : eq[0];
       if (A.out_q != nullptr) A.out_q[i] = A.accumulate ? A.out_q[i] + eq[1] : eq[1];

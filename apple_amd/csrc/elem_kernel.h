@@ -31,6 +31,7 @@
 
 #include "internal.h"
 #include "tetmath.h"
+#include "flatsum.h"
 #include "persist.h"
 #include "solve_state.h"
 
@@ -89,11 +90,16 @@ struct alignas(2 * sizeof(T)) Vec2 {
 //   W_DIR    the accepted step: the block forms the new iterate and direction
 //            of its vertices while it stages them, and the slot that comes
 //            first in a vertex's partial run (the owner) writes them to the
-//            other buffer.  Without this the step is a launch of its own
-//            that reads and writes every vertex once more.
+//            other buffer.  As a launch of its own the step took 8.2 us at
+//            64^3 cubes and 3.8 us (the launch) at 10^3; here it adds 4.5 us
+//            to a 20 us pass at 64^3 (the records of a vertex are read once
+//            per block that touches it, 2.3 times) and nothing at 10^3.
 //   W_CGD    the CG direction d = z + beta d, formed and written the same way
 //   W_ACT    the caller's direction, blocks of running instances only
-constexpr unsigned W_TRIAL = 256u, W_DIR = 512u, W_CGD = 1024u, W_ACT = 2048u;
+// W_FUSED with one of them: a single instance's pass that takes the scalar
+// step before it (scalar_step).  A variant of its own: the batches' passes
+// lose 8-15 % to the registers and scalar traffic of that code.
+constexpr unsigned W_TRIAL = 256u, W_DIR = 512u, W_CGD = 1024u, W_ACT = 2048u, W_FUSED = 4096u;
 constexpr unsigned W_SOLVER = W_TRIAL | W_DIR | W_CGD | W_ACT;
 constexpr unsigned W_OUT = 255u;  // the bits tet_eval knows
 constexpr unsigned OWNER_BIT = 0x80000000u;
@@ -105,7 +111,11 @@ struct NoSolve {};
 // three loads each, and the staging loads are what bounds the direction pass).
 template <class R>
 struct SolveArgs {
-  const InstState* st;
+  const InstState* st;  // the states this pass acts on; W_FUSED: those before its scalar step,
+  InstState* out;       // where workgroup 0 keeps those after it,
+  const double* table;  // and the table that the pass before left for it
+  int n_table;
+  Params prm;
   Vec4<double>* x;  // PNCG iterate: two buffers of V (InstState::cur)
   Vec4<R>* p;       // PNCG / CG direction: two buffers of V
   const Vec4<R>* g;   // two buffers of V: g - f, 0 on fixed DOFs
@@ -118,6 +128,24 @@ struct SolveArgs {
   size_t V;
   int n_iso;      // (first launch of a pass only)
   int filter;     // visit only blocks of active instances (batches)
+};
+
+// The scalars of an instance that a pass needs, in scalar registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uni(double v) {
+  const long long b = __builtin_bit_cast(long long, v);
+  const int lo = __builtin_amdgcn_readfirstlane((int)(b & 0xffffffffll));
+  const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+}
+
+struct InstScalars {
+  double alpha, alpha_commit, beta, pmean;
+  int act_eval, commit, act_dir, cur;
+  InstScalars() = default;
+  __device__ explicit InstScalars(const InstState& s)
+      : alpha(uni(s.alpha)), alpha_commit(uni(s.alpha_commit)), beta(uni(s.beta)), pmean(uni(s.pmean)),
+        act_eval(uni(s.act_eval)), commit(uni(s.commit)), act_dir(uni(s.act_dir)), cur(uni(s.cur)) {}
 };
 
 // An accepted step: x += alpha_commit p, p = -P g + beta p with the Jacobi
@@ -134,7 +162,8 @@ struct Step {
   const Vec4<R>* P;
   Vec4<double>* x1;
   Vec4<R>* p1;
-  __device__ Step(const SolveArgs<R>& S, const InstState& st)
+  template <class State>
+  __device__ Step(const SolveArgs<R>& S, const State& st)
       : a(st.alpha_commit), beta((R)st.beta), ipm(R(1) / (R)st.pmean), dir(st.act_dir != 0),
         x0(S.x + (st.cur ? (size_t)0 : S.V)), p0(S.p + (st.cur ? (size_t)0 : S.V)),
         g(S.g + (st.cur ? S.V : (size_t)0)), P(S.P), x1(S.x + (st.cur ? S.V : (size_t)0)),
@@ -298,13 +327,13 @@ __device__ __forceinline__ void step_vertex(const Step<R>& t, unsigned v, bool o
 
 // ... at the vertices no tet touches (no block stages them)
 template <class R>
-__device__ __forceinline__ void step_isolated(const SolveArgs<R>& S) {
+__device__ __forceinline__ void step_isolated(const SolveArgs<R>& S, const InstState* st) {
   for (int k = (int)blockIdx.x * NTH + (int)threadIdx.x; k < S.n_iso; k += (int)gridDim.x * NTH) {
-    const InstState& st = S.st[S.iso_inst[k]];
-    if (st.commit == 0) continue;
+    const InstState& s = st[S.iso_inst[k]];
+    if (s.commit == 0) continue;
     Vec4<double> u;
     Vec4<R> d;
-    step_vertex(Step<R>(S, st), (unsigned)S.iso[k], true, u, d);
+    step_vertex(Step<R>(S, s), (unsigned)S.iso[k], true, u, d);
   }
 }
 
@@ -316,7 +345,8 @@ struct Direction {
   const Vec4<R>* z;
   const Vec4<R>* d0;
   Vec4<R>* d1;
-  __device__ Direction(const SolveArgs<R>& S, const InstState& st)
+  template <class State>
+  __device__ Direction(const SolveArgs<R>& S, const State& st)
       : beta((R)st.beta), z(S.z), d0(S.p + (st.cur ? (size_t)0 : S.V)), d1(S.p + (st.cur ? S.V : (size_t)0)) {}
 };
 
@@ -330,13 +360,40 @@ __device__ __forceinline__ void direction_vertex(const Direction<R>& t, unsigned
 }
 
 template <class R>
-__device__ __forceinline__ void direction_isolated(const SolveArgs<R>& S) {
+__device__ __forceinline__ void direction_isolated(const SolveArgs<R>& S, const InstState* st) {
   for (int k = (int)blockIdx.x * NTH + (int)threadIdx.x; k < S.n_iso; k += (int)gridDim.x * NTH) {
-    const InstState& st = S.st[S.iso_inst[k]];
-    if (st.act_eval == 0) continue;
+    const InstState& s = st[S.iso_inst[k]];
+    if (s.act_eval == 0) continue;
     Vec4<R> d;
-    direction_vertex(Direction<R>(S, st), (unsigned)S.iso[k], true, d);
+    direction_vertex(Direction<R>(S, s), (unsigned)S.iso[k], true, d);
   }
+}
+
+// The scalar step before a pass, taken by every workgroup of a single
+// instance's pass for itself.  A kernel of its own for one thread's decision
+// costs a launch and a walk over the table by one CU (4.4 us each in a
+// captured graph); here the pass grows by 1.5-2.3 us.  A PNCG iteration of a
+// 10^3 cube went from 19.7 to 17.9 us, of a 32^3 ARAP cube from 35.5 to 31 us.
+template <unsigned WHAT, class R>
+__device__ __forceinline__ void scalar_step(const SolveArgs<R>& S, InstState* st, double* sm) {
+  static_assert(sizeof(InstState) == 8 * STATE_DOUBLES, "state record");
+  // every load before the first wait: the state (one double per thread) and the table
+  const int t = threadIdx.x;
+  double s_in = 0.0;
+  if (t < STATE_DOUBLES) s_in = reinterpret_cast<const double*>(S.st)[t];
+  if constexpr ((WHAT & W_TRIAL) != 0) {
+    const double q = flat_sum_odd_short<SCAL_TH, NTH>(S.table, S.n_table, sm);
+    if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
+    __syncthreads();
+    if (t == 0) pncg_alpha_step(*st, S.prm, q);
+  } else if constexpr ((WHAT & W_DIR) != 0) {
+    flat_column_sums_short<N_DOTS, SCAL_TH, NTH>(S.table, S.n_table, sm);
+    if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
+    __syncthreads();
+    if (t == 0 && st->act_eval != 0) pncg_scalar_step(*st, S.prm, sm);
+  }
+  __syncthreads();
+  if (blockIdx.x == 0 && t < STATE_DOUBLES) reinterpret_cast<double*>(S.out)[t] = reinterpret_cast<double*>(st)[t];
 }
 
 // SPT: slot items per thread.  A block with nloc slots splits each slot's
@@ -354,6 +411,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   constexpr bool DIR = (WHAT & W_DIR) != 0;
   constexpr bool CGD = (WHAT & W_CGD) != 0;
   constexpr bool SOLVER = (WHAT & W_SOLVER) != 0;
+  constexpr bool FUSED = (WHAT & W_FUSED) != 0;
   static_assert(SOLVER == !std::is_same_v<SOLVE, NoSolve>, "solver passes take SolveArgs");
   constexpr bool HAS_G = (WHAT & W_G) != 0;
   constexpr bool HAS_H = (WHAT & W_H) != 0;
@@ -367,8 +425,11 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   static_assert(NCH <= MAX_CH, "too many channels");
 
   extern __shared__ double smem_d[];
-  double* red = smem_d;                          // wave partials of the block sums
-  X* u_lds = reinterpret_cast<X*>(smem_d + 8);  // 4 per slot (padded)
+  double* red = smem_d;  // wave partials of the block sums
+  // the fused scalar step's state and, before the first block, its table sums
+  InstState* st_lds = reinterpret_cast<InstState*>(smem_d + 8);
+  constexpr int HEAD = 8 + (FUSED ? STATE_DOUBLES : 0);
+  X* u_lds = reinterpret_cast<X*>(smem_d + HEAD);  // 4 per slot (padded)
   R* v_lds = reinterpret_cast<R*>(u_lds + 4 * A.nloc_max);
   R* contrib = v_lds + (NEEDV ? 4 * A.nloc_max : 0);  // [channel group][position][channel in group]
   using PK = Pack<NCHA>;
@@ -400,10 +461,17 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   // only those of still-active instances.
   const int n_cand = k0 < nb_x ? (nb_x - k0 + K - 1) / K : 0;
   bool filter = false;
-  if constexpr (SOLVER) {
+  InstScalars single;  // the instance's scalars (FUSED)
+  if constexpr (FUSED) {
+    scalar_step<WHAT>(S, st_lds, smem_d + HEAD);
+    if constexpr (DIR) step_isolated(S, st_lds);
+    if constexpr (CGD) direction_isolated(S, st_lds);
+    single = InstScalars(*st_lds);
+    if ((DIR ? single.commit : single.act_eval) == 0) return;
+  } else if constexpr (SOLVER) {
+    if constexpr (DIR) step_isolated(S, S.st);
+    if constexpr (CGD) direction_isolated(S, S.st);
     filter = S.filter != 0;
-    if constexpr (DIR) step_isolated(S);
-    if constexpr (CGD) direction_isolated(S);
     if (!filter && (DIR ? S.st[0].commit : S.st[0].act_eval) == 0) return;
   }
   // the active-block list (solves only) sits after the contribution buffer
@@ -427,7 +495,15 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         return true;
       },
       [&](const int b, const int bn) {
-      const int inst = A.blk_inst[b];
+      // the scalars of the block's instance
+      const auto& st = [&]() -> const auto& {
+        if constexpr (FUSED)
+          return single;
+        else if constexpr (SOLVER)
+          return S.st[A.blk_inst[b]];
+        else
+          return S;
+      }();
       const int t0 = A.blk_tet_off[b];
       const int nt = A.blk_tet_off[b + 1] - t0;
       const int sb = A.blk_loc_off[b];
@@ -455,7 +531,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       // new iterate and direction for an accepted step)
       const int32_t* gids = A.loc_gid + sb;
       if constexpr (DIR) {
-        const Step<R> step(S, S.st[inst]);
+        const Step<R> step(S, st);
         for (int s = tid; s < nloc; s += NTH) {
           const uint32_t o = at(S.own + sb, (unsigned)s);
           Vec4<X> u4;
@@ -466,7 +542,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         }
         if (!step.dir) return;  // converged at this step: no new direction
       } else if constexpr (CGD) {
-        const Direction<R> dir(S, S.st[inst]);
+        const Direction<R> dir(S, st);
         for (int s = tid; s < nloc; s += NTH) {
           const uint32_t o = at(S.own + sb, (unsigned)s);
           const unsigned v = o & ~OWNER_BIT;
@@ -477,7 +553,6 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4;
         }
       } else if constexpr (TRIAL) {
-        const InstState& st = S.st[inst];
         const double alpha = st.alpha;
         const Vec4<double>* xb = S.x + (st.cur ? S.V : (size_t)0);
         const Vec4<R>* pb = S.p + (st.cur ? S.V : (size_t)0);
@@ -813,8 +888,13 @@ template <unsigned WHAT, class R, class X>
 constexpr size_t smem_bytes_n(int nloc_max, bool filtered) {
   constexpr bool NEEDV = (WHAT & (W_HP | W_HQ | W_MIX | W_MIXA)) != 0;
   constexpr int NCH = ((WHAT & W_G) ? 3 : 0) + ((WHAT & W_H) ? 3 : 0) + ((WHAT & W_HP) ? 3 : 0);
-  size_t n = 8 * sizeof(double) + 4 * (size_t)nloc_max * (sizeof(X) + (NEEDV ? sizeof(R) : 0));
+  size_t n = 4 * (size_t)nloc_max * (sizeof(X) + (NEEDV ? sizeof(R) : 0));
   n += sizeof(R) * (size_t)(NCH > 0 ? Pack<NCH>::NCHP : 0) * 4 * NTH;
+  if ((WHAT & W_FUSED) != 0) {
+    if (n < SUMS_LDS) n = SUMS_LDS;  // the fused scalar step's sums share the window's space
+    n += STATE_DOUBLES * sizeof(double);
+  }
+  n += 8 * sizeof(double);
   if (filtered) n += sizeof(int) * NTH;  // active-block list
   return n;
 }
@@ -850,7 +930,8 @@ constexpr auto pass_kernel() {
 // row of a pass variant in the mesh's grid cache
 constexpr int variant_index(unsigned what) {
   constexpr unsigned v[N_VARIANTS] = {W_E, W_E | W_G | W_H, W_G, W_H, W_HP, W_HQ, W_MIX, W_MIXA, W_MIX | W_MIXA,
-                                      W_E | W_G | W_H | W_TRIAL, W_HQ | W_DIR, W_HP | W_CGD, W_HP | W_ACT};
+                                      W_E | W_G | W_H | W_TRIAL, W_HQ | W_DIR, W_HP | W_CGD, W_HP | W_ACT,
+                                      W_E | W_G | W_H | W_TRIAL | W_FUSED, W_HQ | W_DIR | W_FUSED};
   for (int i = 0; i < N_VARIANTS; ++i)
     if (v[i] == what) return i;
   return -1;

@@ -4,4 +4,6 @@
 namespace apl {
 APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL, float)
 APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL, double)
+APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL | W_FUSED, float)
+APL_SOLVE_PASS(W_E | W_G | W_H | W_TRIAL | W_FUSED, double)
 }  // namespace apl

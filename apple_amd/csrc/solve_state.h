@@ -26,6 +26,22 @@ struct alignas(16) InstState {
       ls_last, cur;
 };
 
+constexpr int STATE_DOUBLES = sizeof(InstState) / 8;
+
+// threads whose order the sums over whole tables follow (the scalar kernels
+// run with as many: each sums whole tables of per-block values, so more
+// loads in flight shorten them)
+constexpr int SCAL_TH = 1024;
+
+// A single instance's scalar steps ride in the element pass that follows
+// them up to these table sizes (FUSE_BLOCKS element blocks for the step
+// length, FUSE_VBLOCKS vertex blocks of 16 columns for the decision): every
+// workgroup reads the whole table, so beyond them the launch saved costs
+// more in the L2 than it gives (64^3 cubes, 5,120 blocks: the trial pass grew
+// by 3.8 us, the launch is 4.7 us and the whole solve was slower).
+constexpr int FUSE_BLOCKS = 2048, FUSE_VBLOCKS = 192;
+static_assert(FUSE_BLOCKS <= 4 * SCAL_TH && FUSE_VBLOCKS * N_DOTS <= 4 * SCAL_TH, "short tables (flatsum.h)");
+
 struct Params {
   double rtol, atol, overstep, c1, wolfe_delta, wolfe_eps, beta_max;
   int max_steps, max_backtracking, stall_steps;

@@ -11,13 +11,15 @@
 // differences stop resolving the decrease long before ||g|| reaches 1e-6
 // relative in FP32, the directional-derivative test does not.
 //
-// One iteration is five launches, all with device-side control (no host sync):
+// One iteration, all with device-side control (no host sync):
+//   S2 per-instance: alpha = -gd / pHp
 //   A  element pass at the trial point x + alpha p: energy, gradient, Hdiag
 //   R  vertex pass: sums of shared-vertex partials, masks, FP64 partial dots
 //   S  per-instance scalar step: energy/dot totals, accept/reject, beta, gd
 //   B  element pass: the step x += alpha p, p = -P g + beta p formed while the
 //      blocks stage their vertices, and p^T H p (clamped per tet)
-//   S2 per-instance: alpha = -gd / pHp
+// S2 and S are taken by A's and B's own workgroups for a single instance
+// whose tables are small (FUSE_BLOCKS, FUSE_VBLOCKS), else they are launches.
 // A rejected trial skips B/S2 work (flags) and the next A re-evaluates at
 // the halved step.  K iterations are captured in one HIP graph; the host
 // checks the per-instance status once per graph launch.  Every instance of a
@@ -39,10 +41,6 @@
 #include "tetmath.h"
 
 namespace apl {
-
-// threads of the per-instance scalar kernels: each sums whole tables of
-// per-block values, so more loads in flight shorten them
-constexpr int SCAL_TH = 1024;
 
 // Workgroup sums of the 16 per-thread dots, in a fixed order, to out[0..16).
 // Recursive halving across the wave (offsets 32, 16, 8, 4: each lane keeps
@@ -130,9 +128,10 @@ __global__ __launch_bounds__(NTH) void fill_kernel(R* a, long long n, R v) {
   for (long long i = (long long)blockIdx.x * NTH + threadIdx.x; i < n; i += (long long)gridDim.x * NTH) a[i] = v;
 }
 
+// both copies of the states
 __global__ void solve_init_kernel(InstState* st, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  if (i >= 2 * n) return;
   InstState s{};
   s.pmean = 1.0;
   s.gbest = INFINITY;
@@ -274,38 +273,38 @@ __global__ __launch_bounds__(NTH) void pncg_reduce_kernel(VecArgs<R> A) {
                 [&](int vb) { pncg_reduce_block<R>(A, vb, sm, win); });
 }
 
-// S: per-instance decision, one workgroup per instance
-__global__ __launch_bounds__(SCAL_TH) void pncg_scalar_kernel(InstState* st, Params P, const double* vblk_dots,
-                                                          const int64_t* inst_vblk_off) {
-  __shared__ double sm[(SCAL_TH / 64 + 1) * N_DOTS];
+// S: per-instance decision, one workgroup per instance, from the states `in`
+// to `out`
+__global__ __launch_bounds__(SCAL_TH) void pncg_scalar_kernel(const InstState* in, InstState* out, Params P,
+                                                          const double* vblk_dots, const int64_t* inst_vblk_off) {
+  __shared__ double tot[(SCAL_TH / 64 + 1) * N_DOTS];
   const int i = blockIdx.x;
   // the active flag, the table bounds and the state are independent: all are
   // loaded before the first wait (an inactive instance sums an empty table)
-  const bool act = st[i].act_eval != 0;
+  const bool act = in[i].act_eval != 0;
   const long long vb0 = inst_vblk_off[i], vb1 = inst_vblk_off[i + 1];
   InstState s;
-  if (threadIdx.x == 0) s = st[i];
-  double tot[N_DOTS];
-  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, act ? (vb1 - vb0) * N_DOTS : 0, sm, tot);
-  if (threadIdx.x != 0 || !act) return;
-  pncg_scalar_step(s, P, tot);
-  st[i] = s;
+  if (threadIdx.x == 0) s = in[i];
+  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, act ? (vb1 - vb0) * N_DOTS : 0, tot);
+  if (threadIdx.x != 0) return;
+  if (act) pncg_scalar_step(s, P, tot);
+  out[i] = s;
 }
 
 // S2: alpha from the quadratic form; clears the per-iteration flags
-__global__ __launch_bounds__(SCAL_TH) void pncg_alpha_kernel(InstState* st, Params P, const double* hq,
-                                                         const int64_t* inst_blk_off) {
+__global__ __launch_bounds__(SCAL_TH) void pncg_alpha_kernel(const InstState* in, InstState* out, Params P,
+                                                         const double* hq, const int64_t* inst_blk_off) {
   __shared__ double red[SCAL_TH / 64];
   const int i = blockIdx.x;
   // all loads issued before the first wait, as in pncg_scalar_kernel
-  const bool dir = st[i].act_dir != 0;
+  const bool dir = in[i].act_dir != 0;
   const long long b0 = inst_blk_off[i], b1 = inst_blk_off[i + 1];
   InstState s;
-  if (threadIdx.x == 0) s = st[i];
+  if (threadIdx.x == 0) s = in[i];
   const double q = flat_sum_odd<SCAL_TH>(hq + b0, dir ? b1 - b0 : 0, red);
   if (threadIdx.x != 0) return;
   pncg_alpha_step(s, P, q);
-  st[i] = s;
+  out[i] = s;
 }
 
 // ------------------------------------------------------------------ PCG (adjoint)
@@ -436,7 +435,7 @@ __global__ __launch_bounds__(NTH) void cg_vec_kernel(CgArgs<R> A) {
 // per-instance CG scalars (one thread); stage 0: after DIAG, 1: after
 // PRECOND, 2: after Q, 3: after UPDATE
 __device__ inline void cg_scalar_step(InstState& s, int stage, double rtol, int max_iters,
-                                      const double (&tot)[N_DOTS]) {
+                                      const double* tot) {
   if (stage == 0) {
     s.pmean = tot[D_HCNT] > 0.0 ? tot[D_HSUM] / tot[D_HCNT] : 1.0;
     const double bn = sqrt(tot[D_G2]);
@@ -486,14 +485,13 @@ __device__ inline void cg_scalar_step(InstState& s, int stage, double rtol, int 
 // the CG's scalar stages, one workgroup per instance
 __global__ __launch_bounds__(SCAL_TH) void cg_scalar_kernel(InstState* st, int stage, double rtol, int max_iters,
                                                         const double* vblk_dots, const int64_t* inst_vblk_off) {
-  __shared__ double sm[(SCAL_TH / 64 + 1) * N_DOTS];
+  __shared__ double tot[(SCAL_TH / 64 + 1) * N_DOTS];
   const int i = blockIdx.x;
   const bool act = stage < 2 || st[i].act_eval != 0;  // loaded with the rest, as in pncg_scalar_kernel
   const long long vb0 = inst_vblk_off[i], vb1 = inst_vblk_off[i + 1];
   InstState s;
   if (threadIdx.x == 0) s = st[i];
-  double tot[N_DOTS];
-  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, act ? (vb1 - vb0) * N_DOTS : 0, sm, tot);
+  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, act ? (vb1 - vb0) * N_DOTS : 0, tot);
   if (threadIdx.x != 0 || !act) return;
   cg_scalar_step(s, stage, rtol, max_iters, tot);
   st[i] = s;
@@ -517,7 +515,7 @@ struct apl_solver {
   int32_t* iso = nullptr;  // vertices without tets, then their instances
   int n_iso = 0;
   double* hq = nullptr;    // per element block: quadratic form of the direction
-  InstState* st = nullptr;
+  InstState* st = nullptr;  // states after the step length (n), then after the decision (n)
   hipStream_t cap = nullptr;
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -564,6 +562,9 @@ static SolveArgs<R> solve_args(apl_solver* s, bool cg) {
   apl_mesh* m = s->mesh;
   SolveArgs<R> S;
   S.st = s->st;
+  S.out = nullptr;
+  S.table = nullptr;
+  S.n_table = 0;
   S.x = s->x;
   S.V = (size_t)m->L.V;
   S.z = (const Vec4<R>*)s->cg;
@@ -611,14 +612,36 @@ static int pncg_iteration(apl_solver* s, const void* mu, const void* lam, const 
                           const Params& P, int grid, hipStream_t st) {
   apl_mesh* m = s->mesh;
   const VecArgs<R> A = vec_args<R>(s, fext, mask);
-  const SolveArgs<R> S = solve_args<R>(s, false);
+  SolveArgs<R> S = solve_args<R>(s, false);
+  S.prm = P;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   const unsigned ni = (unsigned)m->L.n_inst;
-  if (launch_solve_pass<PASS_TRIAL, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st)) return -1;
+  InstState *sa = s->st, *sb = s->st + ni;  // after the step length, after the decision
+  const bool single = ni == 1 && m->L.nblocks > 0;
+  // step length, trial pass
+  int rc = 0;
+  if (single && m->L.nblocks <= FUSE_BLOCKS) {
+    S.st = sb, S.out = sa;
+    S.table = s->hq, S.n_table = (int)m->L.nblocks;
+    rc = launch_solve_pass<PASS_TRIAL | W_FUSED, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+  } else {
+    hipLaunchKernelGGL(pncg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sb, sa, P, s->hq, m->d.inst_blk_off);
+    S.st = sa;
+    rc = launch_solve_pass<PASS_TRIAL, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+  }
+  if (rc) return -1;
   if (nvb) hipLaunchKernelGGL((pncg_reduce_kernel<R>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(pncg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, s->st, P, m->d.vblk_dots, m->d.inst_vblk_off);
-  if (launch_solve_pass<PASS_DIR, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st)) return -1;
-  hipLaunchKernelGGL(pncg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, s->st, P, s->hq, m->d.inst_blk_off);
+  // decision, direction pass
+  if (single && nvb <= FUSE_VBLOCKS) {
+    S.st = sa, S.out = sb;
+    S.table = m->d.vblk_dots, S.n_table = (int)nvb * N_DOTS;
+    rc = launch_solve_pass<PASS_DIR | W_FUSED, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+  } else {
+    hipLaunchKernelGGL(pncg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sa, sb, P, m->d.vblk_dots, m->d.inst_vblk_off);
+    S.st = sb;
+    rc = launch_solve_pass<PASS_DIR, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+  }
+  if (rc) return -1;
   APL_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -674,7 +697,7 @@ static int pncg_begin_t(apl_solver* s, const void* mu, const void* lam, void* x,
   const Params P = to_params(prm);
   const int K = prm->iters_per_launch > 0 ? prm->iters_per_launch : 16;
   // reset state and work vectors (p and g_cur must start at zero)
-  hipLaunchKernelGGL(solve_init_kernel, dim3((n + 255) / 256), dim3(256), 0, st, s->st, n);
+  hipLaunchKernelGGL(solve_init_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, st, s->st, n);
   const long long nv = m->L.V;
   if (fill<R>((R*)s->p, 4 * nv, R(0), st) || fill<R>((R*)s->g, 4 * nv, R(0), st)) return -1;
   APL_CHECK_HIP(hipGetLastError());
@@ -688,6 +711,8 @@ static int pncg_begin_t(apl_solver* s, const void* mu, const void* lam, void* x,
   // occupancy-derived grids are queried (and cached) outside any capture
   solve_pass_grid<PASS_TRIAL, R>(m, s->material);
   solve_pass_grid<PASS_DIR, R>(m, s->material);
+  solve_pass_grid<PASS_TRIAL | W_FUSED, R>(m, s->material);
+  solve_pass_grid<PASS_DIR | W_FUSED, R>(m, s->material);
   // cached graph of K iterations for these pointers and parameters
   bool use_graph = prm->use_graph != 0;
   if (use_graph) {
@@ -745,7 +770,8 @@ static int pncg_begin_t(apl_solver* s, const void* mu, const void* lam, void* x,
 
 // the instances' states on the host (waits for the stream)
 static int read_states(apl_solver* s, hipStream_t st) {
-  APL_CHECK_HIP(hipMemcpyAsync(s->host_st, s->st, (size_t)s->mesh->L.n_inst * sizeof(InstState), hipMemcpyDeviceToHost, st));
+  const size_t n = (size_t)s->mesh->L.n_inst;
+  APL_CHECK_HIP(hipMemcpyAsync(s->host_st, s->st + n, n * sizeof(InstState), hipMemcpyDeviceToHost, st));
   APL_CHECK_HIP(hipStreamSynchronize(st));
   return 0;
 }
@@ -756,7 +782,7 @@ static int copy_iterate(apl_solver* s, void* out, hipStream_t st) {
   apl_mesh* m = s->mesh;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   if (nvb == 0) return 0;
-  hipLaunchKernelGGL((iterate_kernel<R>), dim3(nvb), dim3(NTH), 0, st, s->st, m->d.vblk_off, m->d.vblk_inst, s->x,
+  hipLaunchKernelGGL((iterate_kernel<R>), dim3(nvb), dim3(NTH), 0, st, s->st + m->L.n_inst, m->d.vblk_off, m->d.vblk_inst, s->x,
                      (size_t)m->L.V, (R*)out);
   APL_CHECK_HIP(hipGetLastError());
   return 0;
@@ -860,7 +886,7 @@ static CgArgs<R> cg_args(apl_solver* s, const void* rhs, void* y, const uint8_t*
   A.t = base + 3 * nv;
   A.tout = A.t;
   A.vblk_dots = m->d.vblk_dots;
-  A.st = s->st;
+  A.st = s->st + m->L.n_inst;
   A.V = (size_t)m->L.V;
   A.nvblk = (int)s->mesh->L.vblk_inst.size();
   A.filter = s->mesh->L.n_inst > 1 ? 1 : 0;
@@ -874,7 +900,8 @@ static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const vo
   apl_mesh* m = s->mesh;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   const unsigned ni = (unsigned)m->L.n_inst;
-  const SolveArgs<R> S = solve_args<R>(s, true);
+  SolveArgs<R> S = solve_args<R>(s, true);
+  S.st = A.st;
   if (launch_solve_pass<PASS_CGD, R>(m, s->material, mu, lam, x, nullptr, S, 0, st)) return -1;
   if (A.normal) {
     // q = H (H d): t = H d with fixed DOFs zeroed, then the pass on t
@@ -884,10 +911,10 @@ static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const vo
     if (launch_solve_pass<PASS_ACT, R>(m, s->material, mu, lam, x, A.t, S, 0, st)) return -1;
   }
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_Q>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, s->st, 2, rtol, max_iters, m->d.vblk_dots,
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, A.st, 2, rtol, max_iters, m->d.vblk_dots,
                      m->d.inst_vblk_off);
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_UPDATE>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, s->st, 3, rtol, max_iters, m->d.vblk_dots,
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, A.st, 3, rtol, max_iters, m->d.vblk_dots,
                      m->d.inst_vblk_off);
   APL_CHECK_HIP(hipGetLastError());
   return 0;
@@ -901,7 +928,7 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   const int n = (int)m->L.n_inst;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   CgArgs<R> A = cg_args<R>(s, rhs, y, mask);
-  hipLaunchKernelGGL(solve_init_kernel, dim3((n + 255) / 256), dim3(256), 0, st, s->st, n);
+  hipLaunchKernelGGL(solve_init_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, st, s->st, n);
   if (normal) {
     // the normal equations' right-hand side H b (b with fixed DOFs zeroed),
     // kept by the solver; the CG then runs on it
@@ -919,10 +946,10 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   if (fill<R>(A.hd, 3 * (long long)m->L.V, R(0), st)) return -1;
   if (launch_elem(m, s->material, W_H, mu, lam, x, nullptr, nullptr, A.hd, 0, st)) return -1;
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_DIAG>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, s->st, 0, rtol, max_iters, m->d.vblk_dots,
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, A.st, 0, rtol, max_iters, m->d.vblk_dots,
                      m->d.inst_vblk_off);
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_PRECOND>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, s->st, 1, rtol, max_iters, m->d.vblk_dots,
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, A.st, 1, rtol, max_iters, m->d.vblk_dots,
                      m->d.inst_vblk_off);
   APL_CHECK_HIP(hipGetLastError());
   solve_pass_grid<PASS_CGD, R>(m, s->material);
@@ -1027,7 +1054,7 @@ int apl_solver_create(apl_mesh* m, int material, apl_solver** out) {
     total += (bytes + 255) / 256 * 256;
     return off;
   };
-  const size_t o_st = part((size_t)n * sizeof(InstState)), o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)),
+  const size_t o_st = part(2 * (size_t)n * sizeof(InstState)), o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)),
                o_p = part(2 * nv * 4 * rs), o_g = part(3 * nv * 4 * rs), o_cg = part(3 * nv * 4 * rs),
                o_vecs = part(N_VECS * nv * 3 * rs),
                o_own = part((size_t)std::max<int64_t>(m->L.n_slots, 1) * sizeof(uint32_t)),
