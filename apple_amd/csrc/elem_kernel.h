@@ -32,6 +32,7 @@
 #include "internal.h"
 #include "tetmath.h"
 #include "flatsum.h"
+#include "lanes.h"
 #include "persist.h"
 #include "solve_state.h"
 
@@ -169,46 +170,6 @@ struct Step {
         g(S.g + (st.cur ? S.V : (size_t)0)), P(S.P), x1(S.x + (st.cur ? S.V : (size_t)0)),
         p1(S.p + (st.cur ? S.V : (size_t)0)) {}
 };
-
-// Cross-lane moves by DPP (VALU; no LDS round trip as with ds_bpermute).
-// Lanes whose DPP source does not exist (row_shr at a row start, rows the
-// row mask leaves out) read `old` = 0.
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, false));
-}
-template <int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, ROW_MASK, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xF, false);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-template <class T, int CTRL, int ROW_MASK = 0xF>
-__device__ __forceinline__ T dpp(T v) {
-  if constexpr (sizeof(T) == 4)
-    return dpp_f32<CTRL, ROW_MASK>(v);
-  else
-    return dpp_f64<CTRL, ROW_MASK>(v);
-}
-// gfx9 DPP controls
-constexpr int DPP_QUAD_XOR1 = 0xB1;  // quad_perm [1,0,3,2]: the partner lane ^ 1
-constexpr int DPP_QUAD_XOR2 = 0x4E;  // quad_perm [2,3,0,1]: the partner lane ^ 2
-constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114, DPP_ROW_SHR8 = 0x118;
-constexpr int DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;
-
-// Sum over the 64 lanes of a wave by a fixed DPP tree: prefix sums within
-// each row of 16 lanes, then row 0's total into row 1 and row 2's into
-// row 3, then lane 31's into rows 2-3.  The total is in lane 63.
-__device__ inline double wave_sum(double v) {
-  v += dpp_f64<DPP_ROW_SHR1>(v);
-  v += dpp_f64<DPP_ROW_SHR2>(v);
-  v += dpp_f64<DPP_ROW_SHR4>(v);
-  v += dpp_f64<DPP_ROW_SHR8>(v);
-  v += dpp_f64<DPP_ROW_BCAST15, 0xA>(v);
-  v += dpp_f64<DPP_ROW_BCAST31, 0xC>(v);
-  return v;
-}
 
 // Element i of a uniform base pointer through a 32-bit byte offset: maps to
 // the scalar-base + vector-offset load/store form (no per-lane 64-bit
@@ -382,15 +343,24 @@ __device__ __forceinline__ void scalar_step(const SolveArgs<R>& S, InstState* st
   double s_in = 0.0;
   if (t < STATE_DOUBLES) s_in = reinterpret_cast<const double*>(S.st)[t];
   if constexpr ((WHAT & W_TRIAL) != 0) {
+    if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
     const double q = flat_sum_odd_short<SCAL_TH, NTH>(S.table, S.n_table, sm);
-    if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
-    __syncthreads();
-    if (t == 0) pncg_alpha_step(*st, S.prm, q);
+    if (t == 0) {
+      InstState s = *st;
+      pncg_alpha_step(s, S.prm, q);
+      *st = s;
+    }
   } else if constexpr ((WHAT & W_DIR) != 0) {
-    flat_column_sums_short<N_DOTS, SCAL_TH, NTH>(S.table, S.n_table, sm);
     if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
-    __syncthreads();
-    if (t == 0 && st->act_eval != 0) pncg_scalar_step(*st, S.prm, sm);
+    flat_column_sums_short<N_DOTS, SCAL_TH, NTH>(S.table, S.n_table, sm);
+    if (t == 0) {
+      InstState s = *st;
+      double tot[N_DOTS];
+#pragma unroll
+      for (int k = 0; k < N_DOTS; ++k) tot[k] = sm[k];
+      if (s.act_eval != 0) pncg_scalar_step(s, S.prm, tot);
+      *st = s;
+    }
   }
   __syncthreads();
   if (blockIdx.x == 0 && t < STATE_DOUBLES) reinterpret_cast<double*>(S.out)[t] = reinterpret_cast<double*>(st)[t];
@@ -462,7 +432,19 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   const int n_cand = k0 < nb_x ? (nb_x - k0 + K - 1) / K : 0;
   bool filter = false;
   InstScalars single;  // the instance's scalars (FUSED)
+  // FUSED: the first block's tables, records and slot vertices are loaded
+  // before the scalar step, whose sums and barriers hide their latency
+  int pre_b = -1;
+  uint32_t pre_o = 0u;
+  TetRec<R> pre_rec;
   if constexpr (FUSED) {
+    if (n_cand > 0) {
+      pre_b = xcd_block(k0);
+      const int t0 = A.blk_tet_off[pre_b], sb = A.blk_loc_off[pre_b];
+      if (tid < A.blk_tet_off[pre_b + 1] - t0) load_rec<MAT>(block_res<MAT>(A, t0), (unsigned)tid, pre_rec);
+      if (tid < A.blk_loc_off[pre_b + 1] - sb)
+        pre_o = TRIAL ? (uint32_t)at(A.loc_gid + sb, (unsigned)tid) : at(S.own + sb, (unsigned)tid);
+    }
     scalar_step<WHAT>(S, st_lds, smem_d + HEAD);
     if constexpr (DIR) step_isolated(S, st_lds);
     if constexpr (CGD) direction_isolated(S, st_lds);
@@ -525,7 +507,10 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       // two global-load latencies overlap
       const BlockRes br = block_res<MAT>(A, t0);
       TetRec<R> rec;
-      if (tid < nt) load_rec<MAT>(br, (unsigned)tid, rec);
+      if (FUSED && b == pre_b)
+        rec = pre_rec;
+      else if (tid < nt)
+        load_rec<MAT>(br, (unsigned)tid, rec);
 
       // stage the block's vertex window (u = x + alpha p for a trial point; the
       // new iterate and direction for an accepted step)
@@ -533,7 +518,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       if constexpr (DIR) {
         const Step<R> step(S, st);
         for (int s = tid; s < nloc; s += NTH) {
-          const uint32_t o = at(S.own + sb, (unsigned)s);
+          const uint32_t o = FUSED && b == pre_b && s == tid ? pre_o : at(S.own + sb, (unsigned)s);
           Vec4<X> u4;
           Vec4<R> v4;
           step_vertex(step, o & ~OWNER_BIT, (o & OWNER_BIT) != 0, u4, v4);
@@ -557,7 +542,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         const Vec4<double>* xb = S.x + (st.cur ? S.V : (size_t)0);
         const Vec4<R>* pb = S.p + (st.cur ? S.V : (size_t)0);
         for (int s = tid; s < nloc; s += NTH) {
-          const size_t v = (size_t)at(gids, (unsigned)s);
+          const size_t v = FUSED && b == pre_b && s == tid ? (size_t)pre_o : (size_t)at(gids, (unsigned)s);
           Vec4<double> u4 = xb[v];
           const Vec4<R> p4 = pb[v];
 #pragma unroll

@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "lanes.h"
+
 namespace apl {
 
 // LDS bytes the sums below may need
@@ -64,8 +66,11 @@ __device__ inline void flat_column_sums_short(const double* __restrict__ p, int 
 #pragma unroll
   for (int m = 0; m < M; ++m) {
     double s = (v[m][0] + v[m][1]) + (v[m][2] + v[m][3]);
-#pragma unroll
-    for (int off = 32; off >= W; off >>= 1) s += __shfl_down(s, off, 64);
+    s = add_xor<32>(s);
+    if constexpr (W <= 16) s = add_xor<16>(s);
+    if constexpr (W <= 8) s = add_xor<8>(s);
+    if constexpr (W <= 4) s = add_xor<4>(s);
+    if constexpr (W <= 2) s = add_xor<2>(s);
     if (lane < W) sm[(1 + w + m * (NT / 64)) * W + lane] = s;
   }
   __syncthreads();
@@ -125,15 +130,13 @@ __device__ inline double flat_sum_odd_short(const double* __restrict__ p, int n,
       v[u] = f < n ? p[f] : 0.0;
     }
     double s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-#pragma unroll
-    for (int off = 16; off >= 1; off >>= 1) s += __shfl_down(s, off, 32);
+    s = add_xor<1>(add_xor<2>(add_xor<4>(add_xor<8>(add_xor<16>(s)))));
     if ((t & 31) == 0) sm[(t >> 5) + m * (NT / 32)] = s;
   }
   __syncthreads();
   double r = 0.0;
 #pragma unroll
   for (int i = 0; i < H / 32; ++i) r += sm[i];
-  __syncthreads();
   return r;
 }
 

@@ -35,6 +35,7 @@
 #include "elem_solve.h"
 #include "internal.h"
 #include "flatsum.h"
+#include "lanes.h"
 #include "solve_state.h"
 #include "persist.h"
 #include "vsum.h"
@@ -46,27 +47,24 @@ namespace apl {
 // Recursive halving across the wave (offsets 32, 16, 8, 4: each lane keeps
 // half of its entries and adds its partner's copy of them) leaves dot
 // lane / 4 in lanes 4j..4j+3; two more exchanges complete those sums, and
-// the waves are added in order.  17 shuffles instead of 16 x 6.
-template <int HALF, int OFF>
-__device__ __forceinline__ void halving_step(double (&v)[N_DOTS], int lane) {
-  const bool up = (lane & OFF) != 0;
-#pragma unroll
-  for (int k = 0; k < HALF; ++k) {
-    const double send = up ? v[k] : v[k + HALF];
-    const double keep = up ? v[k + HALF] : v[k];
-    v[k] = keep + __shfl_xor(send, OFF, 64);
-  }
-}
-
+// the waves are added in order.  17 exchanges instead of 16 x 6.
 __device__ inline void block_dots(double (&v)[N_DOTS], double* sm, double* out) {
   static_assert(N_DOTS == 16, "halving tree is written for 16 dots");
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  halving_step<8, 32>(v, lane);
-  halving_step<4, 16>(v, lane);
-  halving_step<2, 8>(v, lane);
-  halving_step<1, 4>(v, lane);
-  v[0] += __shfl_xor(v[0], 2, 64);
-  v[0] += __shfl_xor(v[0], 1, 64);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = swap_add<32>(v[k], v[k + 8]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = swap_add<16>(v[k], v[k + 4]);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const bool up = (lane & 8) != 0;
+    v[k] = (up ? v[k + 2] : v[k]) + xor_lane<8>(up ? v[k] : v[k + 2]);
+  }
+  {
+    const bool up = (lane & 4) != 0;
+    v[0] = (up ? v[1] : v[0]) + xor_lane<4>(up ? v[0] : v[1]);
+  }
+  v[0] = add_xor<1>(add_xor<2>(v[0]));
   if ((lane & 3) == 0) sm[w * N_DOTS + (lane >> 2)] = v[0];
   __syncthreads();
   if ((int)threadIdx.x < N_DOTS) {
@@ -81,14 +79,13 @@ __device__ inline void block_dots(double (&v)[N_DOTS], double* sm, double* out) 
 // instance's blocks split into equal consecutive runs, one per vertex block
 // (both counted from the instance's start, so a batch sums the same way as
 // the instance alone).
-__device__ inline void energy_share(const double* blk_red, const int64_t* inst_blk_off,
-                                    const int64_t* inst_vblk_off, int inst, int vb, double& acc) {
-  const long long b0 = inst_blk_off[inst], nb = inst_blk_off[inst + 1] - b0;
-  const long long vb0 = inst_vblk_off[inst], nvb = inst_vblk_off[inst + 1] - vb0;
+__device__ inline double energy_share(const double* blk_red, long long b0, long long nb, long long nvb, long long vb) {
   const long long per = (nb + nvb - 1) / nvb;
-  const long long lo = b0 + (vb - vb0) * per;
+  const long long lo = b0 + vb * per;
   const long long hi = lo + per < b0 + nb ? lo + per : b0 + nb;
+  double acc = 0.0;
   for (long long b = lo + threadIdx.x; b < hi; b += NTH) acc += blk_red[RED_STRIDE * b];
+  return acc;
 }
 
 // Persistent loop of a vector kernel over its vertex blocks blockIdx.x +
@@ -120,7 +117,7 @@ struct VecArgs {
   const InstState* st;
   size_t V;  // vertices: the pairs' second buffers start here
   int nvblk;   // vertex blocks of the mesh
-  int filter;  // visit only blocks of active instances (batches)
+  int nblocks;  // element blocks of the mesh
 };
 
 template <class R>
@@ -185,45 +182,70 @@ __global__ __launch_bounds__(NTH) void isolated_kernel(const int32_t* vblk_off, 
 
 // R: vertex sums of the slot partials + FP64 partial dots of one vertex
 // block (one DOF per thread and stride, coalesced), plus the block's share of
-// the instance's element-block energies
-template <class R>
+// the instance's element-block energies.  What bounds it is the chain of
+// dependent loads: offsets -> partials -> sums -> dots, with the states and
+// the vertex records beside it; every load is started before the first wait
+// of that chain, and the lane exchanges of the dots stay in the VALU.  Per
+// launch 7.4 -> 5.9 us at 10^3 cubes, 8.2 -> 6.5 us at 32^3; at 64^3 (49 MB)
+// 13.3 us as before.  SINGLE (one instance): the block's vertices, its
+// instance and its share of the energies follow from its number, so the chain
+// has no table look-ups before the offsets.  Five waves per SIMD (96 VGPRs)
+// keep the 64^3 mesh's 1,073 workgroups in one round.
+template <class R, bool SINGLE>
 __device__ inline void pncg_reduce_block(const VecArgs<R>& A, const int vb, double* sm, R* win) {
-  const int inst = A.vblk_inst[vb];
+  const int inst = SINGLE ? 0 : A.vblk_inst[vb];
   const InstState& st = A.st[inst];
-  if (st.act_eval == 0) return;
-  const int v0 = A.vblk_off[vb], v1 = A.vblk_off[vb + 1];
+  const int v0 = SINGLE ? vb * NTH : A.vblk_off[vb];
+  const int v1 = SINGLE ? min(v0 + NTH, (int)A.V) : A.vblk_off[vb + 1];
   const int i0 = 3 * v0, i1 = 3 * v1;
+  // the partials' window first (its loads start a chain), then the energies
+  // and the records, which are needed last
+  VertexSums<R, 6, NTH> vs{A.vtx_slot_off, A.partial, win};
+  typename VertexSums<R, 6, NTH>::template Window<12> w;
+  vs.fetch(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R), w);
+  int k0[DOF_PER_THREAD], k1[DOF_PER_THREAD];
+#pragma unroll
+  for (int j = 0; j < DOF_PER_THREAD; ++j) {
+    const int i = i0 + (int)threadIdx.x + j * NTH;
+    k0[j] = k1[j] = 0;
+    if (i < i1) {
+      k0[j] = A.vtx_slot_off[i / 3];
+      k1[j] = A.vtx_slot_off[i / 3 + 1];
+    }
+  }
+  double e_share;
+  if constexpr (SINGLE) {
+    e_share = energy_share(A.blk_red, 0, A.nblocks, A.nvblk, vb);
+  } else {
+    const long long b0 = A.inst_blk_off[inst], vb0 = A.inst_vblk_off[inst];
+    e_share = energy_share(A.blk_red, b0, A.inst_blk_off[inst + 1] - b0, A.inst_vblk_off[inst + 1] - vb0, vb - vb0);
+  }
+  if (SINGLE && st.act_eval == 0) return;  // (batches visit active instances only)
   const double alpha = st.alpha;
   // the committed point's buffers, and where the trial's gradient goes
   const Vec4<double>* x = A.x + (st.cur ? A.V : (size_t)0);
   const Vec4<R>* p = A.p + (st.cur ? A.V : (size_t)0);
   const Vec4<R>* gc0 = A.g + (st.cur ? A.V : (size_t)0);
   Vec4<R>* gt1 = A.g + (st.cur ? (size_t)0 : A.V);
-  // per-DOF inputs, loaded before the partial window so the loads overlap
-  int k0[DOF_PER_THREAD], k1[DOF_PER_THREAD];
   double xv[DOF_PER_THREAD];
   R pv[DOF_PER_THREAD], gcv[DOF_PER_THREAD], fv[DOF_PER_THREAD];
-  bool fixed[DOF_PER_THREAD];
+  unsigned mv[DOF_PER_THREAD];
 #pragma unroll
   for (int j = 0; j < DOF_PER_THREAD; ++j) {
     const int i = i0 + (int)threadIdx.x + j * NTH;
-    k0[j] = k1[j] = 0;
     xv[j] = 0.0;
     pv[j] = gcv[j] = fv[j] = R(0);
-    fixed[j] = true;
+    mv[j] = 0u;
     if (i < i1) {
       const int v = i / 3, c = i - 3 * v;
-      k0[j] = A.vtx_slot_off[v];
-      k1[j] = A.vtx_slot_off[v + 1];
       xv[j] = x[v].v[c];
       pv[j] = p[v].v[c];
       gcv[j] = gc0[v].v[c];
-      fv[j] = A.fext != nullptr ? A.fext[i] : R(0);
-      fixed[j] = A.mask != nullptr && ((A.mask[v] >> c) & 1u) != 0;
+      if (A.fext != nullptr) fv[j] = A.fext[i];
+      if (A.mask != nullptr) mv[j] = A.mask[v];
     }
   }
-  VertexSums<R, 6, NTH> vs{A.vtx_slot_off, A.partial, win};
-  vs.stage(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R));
+  vs.store(w);
   double d[N_DOTS];
 #pragma unroll
   for (int k = 0; k < N_DOTS; ++k) d[k] = 0.0;
@@ -236,11 +258,12 @@ __device__ inline void pncg_reduce_block(const VecArgs<R>& A, const int vb, doub
     vs.sum_dof(k0[j], k1[j], c, gh);
     const double pc = (double)pv[j];
     d[D_EXT] -= (double)fv[j] * (xv[j] + alpha * pc);
-    const R h = gh[1], gf = fixed[j] ? R(0) : gh[0] - fv[j];
-    const R P1 = fixed[j] ? R(0) : (h > R(0) ? R(1) / h : R(-1));
+    const bool fixed = ((mv[j] >> c) & 1u) != 0;
+    const R h = gh[1], gf = fixed ? R(0) : gh[0] - fv[j];
+    const R P1 = fixed ? R(0) : (h > R(0) ? R(1) / h : R(-1));
     gt1[v].v[c] = gf;
     A.P[v].v[c] = P1;
-    if (fixed[j]) continue;
+    if (fixed) continue;
     const double gt = (double)gf;
     const double gc = (double)gcv[j];
     d[D_G2] += gt * gt;
@@ -260,17 +283,17 @@ __device__ inline void pncg_reduce_block(const VecArgs<R>& A, const int vb, doub
     d[D_GCP] += gc * pc;
     d[D_PP] += pc * pc;
   }
-  energy_share(A.blk_red, A.inst_blk_off, A.inst_vblk_off, inst, vb, d[D_E]);
+  d[D_E] = e_share;
   block_dots(d, sm, A.vblk_dots + (long long)vb * N_DOTS);
 }
 
-template <class R>
-__global__ __launch_bounds__(NTH) void pncg_reduce_kernel(VecArgs<R> A) {
+template <class R, bool SINGLE>
+__global__ __launch_bounds__(NTH, sizeof(R) == 4 ? 5 : 4) void pncg_reduce_kernel(VecArgs<R> A) {
   __shared__ double sm[(NTH / 64) * N_DOTS];
   __shared__ R win[VSUM_LDS_BYTES / sizeof(R)];
-  __shared__ int list[NTH];
-  vertex_blocks(A.nvblk, A.filter, list, [&](int vb) { return A.st[A.vblk_inst[vb]].act_eval != 0; },
-                [&](int vb) { pncg_reduce_block<R>(A, vb, sm, win); });
+  __shared__ int list[SINGLE ? 1 : NTH];
+  vertex_blocks(A.nvblk, !SINGLE, list, [&](int vb) { return A.st[A.vblk_inst[vb]].act_eval != 0; },
+                [&](int vb) { pncg_reduce_block<R, SINGLE>(A, vb, sm, win); });
 }
 
 // S: per-instance decision, one workgroup per instance, from the states `in`
@@ -552,7 +575,7 @@ static VecArgs<R> vec_args(apl_solver* s, const void* fext, const uint8_t* mask)
   A.st = s->st;
   A.V = (size_t)m->L.V;
   A.nvblk = (int)m->L.vblk_inst.size();
-  A.filter = m->L.n_inst > 1 ? 1 : 0;
+  A.nblocks = (int)m->L.nblocks;
   return A;
 }
 
@@ -630,7 +653,10 @@ static int pncg_iteration(apl_solver* s, const void* mu, const void* lam, const 
     rc = launch_solve_pass<PASS_TRIAL, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
   }
   if (rc) return -1;
-  if (nvb) hipLaunchKernelGGL((pncg_reduce_kernel<R>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+  if (nvb && ni == 1)
+    hipLaunchKernelGGL((pncg_reduce_kernel<R, true>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+  else if (nvb)
+    hipLaunchKernelGGL((pncg_reduce_kernel<R, false>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
   // decision, direction pass
   if (single && nvb <= FUSE_VBLOCKS) {
     S.st = sa, S.out = sb;

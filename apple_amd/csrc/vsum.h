@@ -39,6 +39,42 @@ struct VertexSums {
     __syncthreads();
   }
 
+  // stage() in two parts, so that a caller's own loads can follow the
+  // window's: fetch() starts the loads of the first N entries of every
+  // thread, store() puts them into LDS (and loads what a longer window has
+  // left).
+  template <int N>
+  struct Window {
+    R v[N];
+    int n, k0;
+  };
+  template <int N>
+  __device__ void fetch(int v0, int v1, int cap, Window<N>& w) {
+    const int k0 = off[v0], k1 = off[v1];
+    k_lo = k0;
+    w.k0 = k0;
+    w.n = (k1 - k0) * NCH;
+    staged = w.n <= cap;
+    if (!staged) w.n = 0;
+    const R* src = partial + (size_t)k0 * NCH;
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int i = (int)threadIdx.x + u * NT;
+      w.v[u] = i < w.n ? src[i] : R(0);
+    }
+  }
+  template <int N>
+  __device__ void store(const Window<N>& w) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int i = (int)threadIdx.x + u * NT;
+      if (i < w.n) lds[i] = w.v[u];
+    }
+    const R* src = partial + (size_t)w.k0 * NCH;
+    for (int i = (int)threadIdx.x + N * NT; i < w.n; i += NT) lds[i] = src[i];
+    __syncthreads();
+  }
+
   // all NCH channels of the vertex whose partial run is [k0, k1)
   __device__ void sum(int k0, int k1, R acc[NCH]) const {
 #pragma unroll
