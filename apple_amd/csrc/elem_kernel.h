@@ -95,7 +95,9 @@ struct alignas(2 * sizeof(T)) Vec2 {
 //            64^3 cubes and 3.8 us (the launch) at 10^3; here it adds 4.5 us
 //            to a 20 us pass at 64^3 (the records of a vertex are read once
 //            per block that touches it, 2.3 times) and nothing at 10^3.
-//   W_CGD    the CG direction d = z + beta d, formed and written the same way
+//   W_CGD    the CG direction d = z + beta d, formed and written the same way;
+//            with W_VQ its d.Hd, so that the update needs no pass of its own
+//            for the step length
 //   W_ACT    the caller's direction, blocks of running instances only
 // W_FUSED with one of them: a single instance's pass that takes the scalar
 // step before it (scalar_step).  A variant of its own: the batches' passes
@@ -361,6 +363,14 @@ __device__ __forceinline__ void scalar_step(const SolveArgs<R>& S, InstState* st
       if (s.act_eval != 0) pncg_scalar_step(s, S.prm, tot);
       *st = s;
     }
+  } else {
+    if (t < STATE_DOUBLES) reinterpret_cast<double*>(st)[t] = s_in;
+    flat_column_sums_short<2, SCAL_TH, NTH>(S.table, S.n_table, sm);
+    if (t == 0) {
+      InstState s = *st;
+      cg_beta_step(s, S.prm.rtol, S.prm.max_steps, sm[0], sm[1]);
+      *st = s;
+    }
   }
   __syncthreads();
   if (blockIdx.x == 0 && t < STATE_DOUBLES) reinterpret_cast<double*>(S.out)[t] = reinterpret_cast<double*>(st)[t];
@@ -390,7 +400,8 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   constexpr bool SCATTER = NCH > 0;
   constexpr int NCHA = NCH > 0 ? NCH : 1;
   constexpr bool NEEDV = (WHAT & (W_HP | W_HQ | W_MIX | W_MIXA)) != 0;
-  constexpr bool RED = (WHAT & (W_E | W_HQ)) != 0;
+  constexpr bool RED_Q = (WHAT & (W_HQ | W_VQ)) != 0;
+  constexpr bool RED = (WHAT & W_E) != 0 || RED_Q;
   constexpr int CS = 4 * NTH;  // channel stride of the contribution buffer
   static_assert(NCH <= MAX_CH, "too many channels");
 
@@ -633,6 +644,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           tet_eval<MAT, WHAT & W_OUT, R>(g, rec.mu, rec.lam, rec.act, u, v, o);
           if constexpr ((WHAT & W_E) != 0) e_acc += o.e;
           if constexpr ((WHAT & W_HQ) != 0) q_acc += o.hq;
+          if constexpr ((WHAT & W_VQ) != 0) q_acc += o.vq;
           if constexpr ((WHAT & W_MIX) != 0) {
             R* oa = A.out_a + t0;
             R* ob = A.out_b + t0;
@@ -796,7 +808,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           const double e = wave_sum((double)e_acc);
           if (lane == 63) red[2 * w] = e;
         }
-        if constexpr ((WHAT & W_HQ) != 0) {
+        if constexpr (RED_Q) {
           const double q = wave_sum((double)q_acc);
           if (lane == 63) red[2 * w + 1] = q;
         }
@@ -805,11 +817,11 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
 #pragma unroll
           for (int col = 0; col < 2; ++col) {
             if (col == 0 && (WHAT & W_E) == 0) continue;
-            if (col == 1 && (WHAT & W_HQ) == 0) continue;
+            if (col == 1 && !RED_Q) continue;
             double r = 0.0;
 #pragma unroll
             for (int ww = 0; ww < NTH / 64; ++ww) r += red[2 * ww + col];
-            if constexpr (DIR)
+            if constexpr (DIR || CGD)
               S.hq[b] = r;
             else
               A.blk_red[(size_t)RED_STRIDE * b + col] = r;
@@ -915,8 +927,9 @@ constexpr auto pass_kernel() {
 // row of a pass variant in the mesh's grid cache
 constexpr int variant_index(unsigned what) {
   constexpr unsigned v[N_VARIANTS] = {W_E, W_E | W_G | W_H, W_G, W_H, W_HP, W_HQ, W_MIX, W_MIXA, W_MIX | W_MIXA,
-                                      W_E | W_G | W_H | W_TRIAL, W_HQ | W_DIR, W_HP | W_CGD, W_HP | W_ACT,
-                                      W_E | W_G | W_H | W_TRIAL | W_FUSED, W_HQ | W_DIR | W_FUSED};
+                                      W_E | W_G | W_H | W_TRIAL, W_HQ | W_DIR, W_HP | W_VQ | W_CGD, W_HP | W_ACT,
+                                      W_E | W_G | W_H | W_TRIAL | W_FUSED, W_HQ | W_DIR | W_FUSED,
+                                      W_HP | W_VQ | W_CGD | W_FUSED};
   for (int i = 0; i < N_VARIANTS; ++i)
     if (v[i] == what) return i;
   return -1;

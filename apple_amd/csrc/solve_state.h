@@ -39,8 +39,10 @@ constexpr int SCAL_TH = 1024;
 // workgroup reads the whole table, so beyond them the launch saved costs
 // more in the L2 than it gives (64^3 cubes, 5,120 blocks: the trial pass grew
 // by 3.8 us, the launch is 4.7 us and the whole solve was slower).
-constexpr int FUSE_BLOCKS = 2048, FUSE_VBLOCKS = 192;
-static_assert(FUSE_BLOCKS <= 4 * SCAL_TH && FUSE_VBLOCKS * N_DOTS <= 4 * SCAL_TH, "short tables (flatsum.h)");
+// FUSE_CG_VBLOCKS: the CG's two columns per vertex block, by the same measure.
+constexpr int FUSE_BLOCKS = 2048, FUSE_VBLOCKS = 192, FUSE_CG_VBLOCKS = 1024;
+static_assert(FUSE_BLOCKS <= 4 * SCAL_TH && FUSE_VBLOCKS * N_DOTS <= 4 * SCAL_TH && FUSE_CG_VBLOCKS * 2 <= 4 * SCAL_TH,
+              "short tables (flatsum.h)");
 
 struct Params {
   double rtol, atol, overstep, c1, wolfe_delta, wolfe_eps, beta_max;
@@ -171,6 +173,51 @@ __device__ inline void pncg_alpha_step(InstState& s, const Params& P, double pHp
   }
   s.commit = 0;
   s.act_dir = 0;
+}
+
+// ---- PCG (adjoint).  State reuse: gd = r.z, gnorm0 = ||b||, gnorm = ||r||,
+// alpha = a, pHp = d.Hd, pmean = mean positive diagonal, f = ||r|| / ||b||,
+// phase = 1 once an update has run.
+
+// before an iteration: from the last update's r.r and r.z the residual, the
+// stop tests and beta
+__device__ inline void cg_beta_step(InstState& s, double rtol, int max_iters, double rr, double rz) {
+  if (s.act_eval == 0) return;
+  if (s.phase == 0) {
+    s.phase = 1;  // the first direction is z (beta 0)
+    return;
+  }
+  const double rn = sqrt(rr);
+  s.gnorm = rn;
+  s.n_steps += 1;
+  s.f = s.gnorm0 > 0.0 ? rn / s.gnorm0 : 0.0;
+  if (rn <= rtol * s.gnorm0) {
+    s.status = APL_PRIMARY_SUCCESS;
+    s.act_eval = 0;
+  } else if (!isfinite(rn)) {
+    s.status = APL_NON_FINITE;
+    s.act_eval = 0;
+  } else if (s.n_steps >= max_iters) {
+    s.status = APL_MAX_STEPS_REACHED;
+    s.act_eval = 0;
+  } else {
+    s.beta = rz / s.gd;
+    s.gd = rz;
+    s.cur ^= 1;  // the next direction is formed in the other buffer
+  }
+}
+
+// after the Hessian-vector pass: the step from d.Hd
+__device__ inline void cg_alpha_step(InstState& s, double dq) {
+  if (s.act_eval == 0) return;
+  s.pHp = dq;
+  if (!(dq > 0.0) || !isfinite(dq)) {
+    s.status = APL_NON_FINITE;
+    s.act_eval = 0;
+    s.alpha = 0.0;
+  } else {
+    s.alpha = s.gd / dq;
+  }
 }
 
 }  // namespace apl

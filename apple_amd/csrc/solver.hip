@@ -331,8 +331,18 @@ __global__ __launch_bounds__(SCAL_TH) void pncg_alpha_kernel(const InstState* in
 }
 
 // ------------------------------------------------------------------ PCG (adjoint)
-// State reuse: gd = r.z, gnorm0 = ||b||, gnorm = ||r||, alpha = a, beta,
-// pHp = d.Hd, pmean = mean positive diagonal, f = ||r|| / ||b||.
+//
+// One iteration is two launches (four for batches and meshes with long
+// tables, whose scalar steps are launches of their own):
+//   H  element pass: beta from the last update's dots (cg_beta_step), the
+//      direction d = z + beta d formed while the blocks stage their vertices,
+//      H d into the slot partials, and d.Hd per block
+//   U  vertex pass: the step from d.Hd (cg_alpha_step), q = H d summed from
+//      the partials, y += a d, r -= a q, z = r / diag, the dots r.r and r.z
+// d.Hd is summed per tet (FP64 over the tets) rather than from q, which would
+// need a vertex pass and a launch of its own between H and U.  An iteration of
+// a 32^3 cube takes 15.8 us (H 9.6, U 5.6; launches 1.6 us each), in five
+// launches it took 28.
 
 template <class R>
 struct CgArgs {
@@ -346,122 +356,123 @@ struct CgArgs {
   R* r;
   Vec4<R>* z;  // padded records, as in SolveArgs
   Vec4<R>* d;  // two buffers (InstState::cur)
-  R* q;
   R* hd;
   R* t;     // normal equations: H d (or the masked right-hand side while it is formed)
   R* tout;  // CG_T / CG_MASKCOPY output
-  double* vblk_dots;
-  InstState* st;
+  double* vblk_dots;  // the initial stages' table, then the update's (2 columns)
+  double* t_dots;     // normal equations: t.t per vertex block
+  const InstState* in;  // the states a stage reads (U with FUSED: before its scalar step)
+  InstState* out;       // U with FUSED: where workgroup 0 keeps those after it
+  const double* hq;     // U with FUSED: d.Hd per element block
   size_t V;
-  int nvblk;   // vertex blocks of the mesh
-  int filter;  // visit only blocks of active instances (batches)
-  int normal;  // CG on the normal equations H^2 y = H b, Jacobi with diag(H)^2
+  int nvblk;    // vertex blocks of the mesh
+  int nblocks;  // element blocks of the mesh
+  int normal;   // CG on the normal equations H^2 y = H b, Jacobi with diag(H)^2
 };
 
-// CG_T: tout = H v summed from the partials, fixed DOFs 0 (no dots);
+// Sums over the workgroup of N per-thread values, to out[0..N): a DPP tree per
+// wave, the waves in order.  sm: NTH / 64 * N doubles.
+template <int N>
+__device__ inline void block_sums(const double (&v)[N], double* sm, double* out) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const double s = wave_sum(v[k]);
+    if (lane == 63) sm[w * N + k] = s;
+  }
+  __syncthreads();
+  if ((int)threadIdx.x < N) {
+    double s = 0.0;
+#pragma unroll
+    for (int ww = 0; ww < NTH / 64; ++ww) s += sm[ww * N + threadIdx.x];
+    out[threadIdx.x] = s;
+  }
+}
+
+// Stages before the iterations, and of the normal equations:
+// CG_DIAG: diag H from its partials, r = b, y = 0, both direction buffers 0
+// CG_PRECOND: z = r / diag
+// CG_T: tout = H v summed from the partials, fixed DOFs 0, and tout.tout
 // CG_MASKCOPY: tout = rhs with fixed DOFs 0
-enum CgStage : int { CG_DIAG = 0, CG_PRECOND = 1, CG_Q = 2, CG_UPDATE = 3, CG_T = 5, CG_MASKCOPY = 6 };
+enum CgStage : int { CG_DIAG = 0, CG_PRECOND = 1, CG_T = 2, CG_MASKCOPY = 3 };
 
 template <class R, int STAGE>
 __device__ inline void cg_vec_block(const CgArgs<R>& A, const int vb, double* sm, R* win) {
-  constexpr bool SUMS = STAGE == CG_DIAG || STAGE == CG_Q || STAGE == CG_T;
-  constexpr bool PRE = STAGE == CG_DIAG || STAGE == CG_PRECOND || STAGE == CG_MASKCOPY;  // before the status
-  const int inst = A.vblk_inst[vb];
-  const InstState& st = A.st[inst];
-  if (!PRE && st.act_eval == 0) return;
-  const Vec4<R>* d = A.d + (st.cur ? A.V : (size_t)0);
+  constexpr bool SUMS = STAGE == CG_DIAG || STAGE == CG_T;
+  const InstState& st = A.in[A.vblk_inst[vb]];
+  if (STAGE == CG_T && st.act_eval == 0) return;
   const int v0 = A.vblk_off[vb], v1 = A.vblk_off[vb + 1];
   const int i0 = 3 * v0, i1 = 3 * v1;
-  double dd[N_DOTS];
-#pragma unroll
-  for (int k = 0; k < N_DOTS; ++k) dd[k] = 0.0;
-  int k0[DOF_PER_THREAD], k1[DOF_PER_THREAD];
-  if constexpr (SUMS) {
-#pragma unroll
-    for (int j = 0; j < DOF_PER_THREAD; ++j) {
-      const int i = i0 + (int)threadIdx.x + j * NTH;
-      k0[j] = k1[j] = 0;
-      if (i < i1) {
-        k0[j] = A.vtx_slot_off[i / 3];
-        k1[j] = A.vtx_slot_off[i / 3 + 1];
-      }
-    }
-  }
   VertexSums<R, 3, NTH> vs{A.vtx_slot_off, A.partial, win};
   if constexpr (SUMS) vs.stage(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R));
+  double d3[3] = {0.0, 0.0, 0.0};
 #pragma unroll
   for (int j = 0; j < DOF_PER_THREAD; ++j) {
     const int i = i0 + (int)threadIdx.x + j * NTH;
     if (i >= i1) continue;
     const int v = i / 3, c = i - 3 * v;
     const bool fixed = A.mask != nullptr && ((A.mask[v] >> c) & 1u) != 0;
-    if constexpr (SUMS) {
-      R s1[1];
-      vs.sum_dof(k0[j], k1[j], c, s1);
-      if constexpr (STAGE == CG_DIAG) {
-        A.hd[i] = s1[0];
-        const R b = fixed ? R(0) : A.rhs[i];
-        A.r[i] = b;
-        A.y[i] = R(0);
-        A.d[v].v[c] = R(0);
-        A.d[A.V + v].v[c] = R(0);
-        A.q[i] = R(0);
-        if (!fixed) {
-          dd[D_G2] += (double)b * (double)b;
-          if (s1[0] > R(0)) {
-            dd[D_HSUM] += (double)s1[0];
-            dd[D_HCNT] += 1.0;
-          }
+    R s1[1];
+    if constexpr (SUMS) vs.sum_dof(A.vtx_slot_off[v], A.vtx_slot_off[v + 1], c, s1);
+    if constexpr (STAGE == CG_DIAG) {
+      A.hd[i] = s1[0];
+      const R b = fixed ? R(0) : A.rhs[i];
+      A.r[i] = b;
+      A.y[i] = R(0);
+      A.d[v].v[c] = R(0);
+      A.d[A.V + v].v[c] = R(0);
+      if (!fixed) {
+        d3[0] += (double)b * (double)b;
+        if (s1[0] > R(0)) {
+          d3[1] += (double)s1[0];
+          d3[2] += 1.0;
         }
-      } else if constexpr (STAGE == CG_T) {
-        A.tout[i] = fixed ? R(0) : s1[0];
-      } else {
-        const R qv = fixed ? R(0) : s1[0];
-        A.q[i] = qv;
-        dd[D_GTP] += (double)d[v].v[c] * (double)qv;
       }
+    } else if constexpr (STAGE == CG_T) {
+      const R t = fixed ? R(0) : s1[0];
+      A.tout[i] = t;
+      d3[0] += (double)t * (double)t;
     } else if constexpr (STAGE == CG_MASKCOPY) {
       A.tout[i] = fixed ? R(0) : A.rhs[i];
-    } else if constexpr (STAGE == CG_PRECOND || STAGE == CG_UPDATE) {
-      const R a = (R)st.alpha;
-      const R pm = (R)st.pmean;
-      R rv = A.r[i];
-      if constexpr (STAGE == CG_UPDATE) {
-        A.y[i] += a * d[v].v[c];
-        rv -= a * A.q[i];
-        A.r[i] = rv;
-      }
-      const R h = A.hd[i];
-      // Jacobi: 1/diag(H), or 1/diag(H)^2 for the normal equations (diag(H^2) >= diag(H)^2)
-      const R hh = h > R(0) ? h : pm;
+    } else {
+      const R rv = A.r[i], h = A.hd[i];
+      const R hh = h > R(0) ? h : (R)st.pmean;
       const R zv = fixed ? R(0) : (A.normal ? rv / (hh * hh) : rv / hh);
       A.z[v].v[c] = zv;
-      dd[D_GPG] += (double)rv * (double)zv;
-      dd[D_G2] += (double)rv * (double)rv;
+      d3[0] += (double)rv * (double)zv;
     }
   }
-  if constexpr (STAGE != CG_T && STAGE != CG_MASKCOPY)
-    block_dots(dd, sm, A.vblk_dots + (long long)vb * N_DOTS);
+  if constexpr (STAGE == CG_T) {
+    const double one[1] = {d3[0]};
+    block_sums<1>(one, sm, A.t_dots + vb);
+  } else if constexpr (STAGE != CG_MASKCOPY) {
+    // (rows of 16 columns, summed by cg_scalar_kernel)
+    block_sums<3>(d3, sm, A.vblk_dots + (long long)vb * N_DOTS);
+  }
+  __syncthreads();
 }
 
 template <class R, int STAGE>
 __global__ __launch_bounds__(NTH) void cg_vec_kernel(CgArgs<R> A) {
-  __shared__ double sm[(NTH / 64) * N_DOTS];
-  constexpr bool SUMS = STAGE == CG_DIAG || STAGE == CG_Q || STAGE == CG_T;
+  __shared__ double sm[(NTH / 64) * 3];
+  constexpr bool SUMS = STAGE == CG_DIAG || STAGE == CG_T;
   __shared__ R win[SUMS ? VSUM_LDS_BYTES / sizeof(R) : 1];
-  __shared__ int list[NTH];
-  constexpr bool ALL = STAGE == CG_DIAG || STAGE == CG_PRECOND || STAGE == CG_MASKCOPY;  // before the status
-  vertex_blocks(A.nvblk, A.filter && !ALL, list, [&](int vb) { return A.st[A.vblk_inst[vb]].act_eval != 0; },
-                [&](int vb) { cg_vec_block<R, STAGE>(A, vb, sm, win); });
+  for (int vb = blockIdx.x; vb < A.nvblk; vb += gridDim.x) cg_vec_block<R, STAGE>(A, vb, sm, win);
 }
 
-// per-instance CG scalars (one thread); stage 0: after DIAG, 1: after
-// PRECOND, 2: after Q, 3: after UPDATE
-__device__ inline void cg_scalar_step(InstState& s, int stage, double rtol, int max_iters,
-                                      const double* tot) {
+// the scalars of the initial stages, one workgroup per instance: 0 after
+// CG_DIAG, 1 after CG_PRECOND
+__global__ __launch_bounds__(SCAL_TH) void cg_scalar_kernel(InstState* st, int stage, const double* vblk_dots,
+                                                        const int64_t* inst_vblk_off) {
+  __shared__ double tot[(SCAL_TH / 64 + 1) * N_DOTS];
+  const int i = blockIdx.x;
+  const long long vb0 = inst_vblk_off[i], vb1 = inst_vblk_off[i + 1];
+  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, (vb1 - vb0) * N_DOTS, tot);
+  if (threadIdx.x != 0) return;
+  InstState s = st[i];
   if (stage == 0) {
-    s.pmean = tot[D_HCNT] > 0.0 ? tot[D_HSUM] / tot[D_HCNT] : 1.0;
-    const double bn = sqrt(tot[D_G2]);
+    s.pmean = tot[2] > 0.0 ? tot[1] / tot[2] : 1.0;
+    const double bn = sqrt(tot[0]);
     s.gnorm0 = bn;
     s.gnorm = bn;
     s.n_steps = 0;
@@ -470,54 +481,134 @@ __device__ inline void cg_scalar_step(InstState& s, int stage, double rtol, int 
     s.act_eval = bn > 0.0 ? 1 : 0;
     s.alpha = 0.0;
     s.beta = 0.0;
-  } else if (stage == 1) {
-    s.gd = tot[D_GPG];
-  } else if (stage == 2) {
-    const double dq = tot[D_GTP];
-    s.pHp = dq;
-    if (!(dq > 0.0) || !isfinite(dq)) {
-      s.status = APL_NON_FINITE;
-      s.act_eval = 0;
-      s.alpha = 0.0;
-    } else {
-      s.alpha = s.gd / dq;
-    }
   } else {
-    const double rz = tot[D_GPG];
-    const double rn = sqrt(tot[D_G2]);
-    s.gnorm = rn;
-    s.n_steps += 1;
-    s.f = s.gnorm0 > 0.0 ? rn / s.gnorm0 : 0.0;
-    if (rn <= rtol * s.gnorm0) {
-      s.status = APL_PRIMARY_SUCCESS;
-      s.act_eval = 0;
-    } else if (!isfinite(rn)) {
-      s.status = APL_NON_FINITE;
-      s.act_eval = 0;
-    } else if (s.n_steps >= max_iters) {
-      s.status = APL_MAX_STEPS_REACHED;
-      s.act_eval = 0;
-    } else {
-      s.beta = rz / s.gd;
-      s.gd = rz;
-      s.cur ^= 1;  // the next direction is formed in the other buffer
-    }
+    s.gd = tot[0];
   }
+  st[i] = s;
 }
 
-// the CG's scalar stages, one workgroup per instance
-__global__ __launch_bounds__(SCAL_TH) void cg_scalar_kernel(InstState* st, int stage, double rtol, int max_iters,
-                                                        const double* vblk_dots, const int64_t* inst_vblk_off) {
-  __shared__ double tot[(SCAL_TH / 64 + 1) * N_DOTS];
+// the iteration's scalar steps as launches, one workgroup per instance
+__global__ __launch_bounds__(SCAL_TH) void cg_beta_kernel(const InstState* in, InstState* out, double rtol, int max_iters,
+                                                      const double* dots, const int64_t* inst_vblk_off) {
+  __shared__ double tot[(SCAL_TH / 64 + 1) * 2];
   const int i = blockIdx.x;
-  const bool act = stage < 2 || st[i].act_eval != 0;  // loaded with the rest, as in pncg_scalar_kernel
+  // all loads issued before the first wait, as in pncg_scalar_kernel
+  const bool act = in[i].act_eval != 0;
   const long long vb0 = inst_vblk_off[i], vb1 = inst_vblk_off[i + 1];
   InstState s;
-  if (threadIdx.x == 0) s = st[i];
-  flat_column_sums<N_DOTS, SCAL_TH>(vblk_dots + vb0 * N_DOTS, act ? (vb1 - vb0) * N_DOTS : 0, tot);
-  if (threadIdx.x != 0 || !act) return;
-  cg_scalar_step(s, stage, rtol, max_iters, tot);
-  st[i] = s;
+  if (threadIdx.x == 0) s = in[i];
+  flat_column_sums<2, SCAL_TH>(dots + 2 * vb0, act ? 2 * (vb1 - vb0) : 0, tot);
+  if (threadIdx.x != 0) return;
+  cg_beta_step(s, rtol, max_iters, tot[0], tot[1]);
+  out[i] = s;
+}
+
+__global__ __launch_bounds__(SCAL_TH) void cg_alpha_kernel(const InstState* in, InstState* out, const double* table,
+                                                       const int64_t* inst_off) {
+  __shared__ double red[SCAL_TH / 64];
+  const int i = blockIdx.x;
+  const bool act = in[i].act_eval != 0;
+  const long long b0 = inst_off[i], b1 = inst_off[i + 1];
+  InstState s;
+  if (threadIdx.x == 0) s = in[i];
+  const double dq = flat_sum_odd<SCAL_TH>(table + b0, act ? b1 - b0 : 0, red);
+  if (threadIdx.x != 0) return;
+  cg_alpha_step(s, dq);
+  out[i] = s;
+}
+
+// U of one vertex block, with the instance's step a and buffer
+template <class R, bool SINGLE>
+__device__ inline void cg_update_block(const CgArgs<R>& A, const int vb, double* sm, R* win, const R a, const R pm,
+                                       const int cur) {
+  const int v0 = SINGLE ? vb * NTH : A.vblk_off[vb];
+  const int v1 = SINGLE ? min(v0 + NTH, (int)A.V) : A.vblk_off[vb + 1];
+  const int i0 = 3 * v0, i1 = 3 * v1;
+  const Vec4<R>* d = A.d + (cur ? A.V : (size_t)0);
+  // as in pncg_reduce_block: every load before the first wait
+  VertexSums<R, 3, NTH> vs{A.vtx_slot_off, A.partial, win};
+  typename VertexSums<R, 3, NTH>::template Window<8> w;
+  vs.fetch(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R), w);
+  int k0[DOF_PER_THREAD], k1[DOF_PER_THREAD];
+  R dv[DOF_PER_THREAD], yv[DOF_PER_THREAD], rv[DOF_PER_THREAD], hv[DOF_PER_THREAD];
+  unsigned mv[DOF_PER_THREAD];
+#pragma unroll
+  for (int j = 0; j < DOF_PER_THREAD; ++j) {
+    const int i = i0 + (int)threadIdx.x + j * NTH;
+    k0[j] = k1[j] = 0;
+    dv[j] = yv[j] = rv[j] = hv[j] = R(0);
+    mv[j] = 0u;
+    if (i < i1) {
+      const int v = i / 3, c = i - 3 * v;
+      k0[j] = A.vtx_slot_off[v];
+      k1[j] = A.vtx_slot_off[v + 1];
+      dv[j] = d[v].v[c];
+      yv[j] = A.y[i];
+      rv[j] = A.r[i];
+      hv[j] = A.hd[i];
+      if (A.mask != nullptr) mv[j] = A.mask[v];
+    }
+  }
+  vs.store(w);
+  double dots[2] = {0.0, 0.0};
+#pragma unroll
+  for (int j = 0; j < DOF_PER_THREAD; ++j) {
+    const int i = i0 + (int)threadIdx.x + j * NTH;
+    if (i >= i1) continue;
+    const int v = i / 3, c = i - 3 * v;
+    const bool fixed = ((mv[j] >> c) & 1u) != 0;
+    R s1[1];
+    vs.sum_dof(k0[j], k1[j], c, s1);
+    A.y[i] = yv[j] + a * dv[j];
+    const R r = rv[j] - a * (fixed ? R(0) : s1[0]);
+    A.r[i] = r;
+    // Jacobi: 1/diag(H), or 1/diag(H)^2 for the normal equations (diag(H^2) >= diag(H)^2)
+    const R hh = hv[j] > R(0) ? hv[j] : pm;
+    const R z = fixed ? R(0) : (A.normal ? r / (hh * hh) : r / hh);
+    A.z[v].v[c] = z;
+    dots[0] += (double)r * (double)r;
+    dots[1] += (double)r * (double)z;
+  }
+  block_sums<2>(dots, sm, A.vblk_dots + 2 * (long long)vb);
+}
+
+// MODE: a batch, a single instance whose scalar step was a launch, or one
+// whose workgroups take the step themselves (FUSE_BLOCKS)
+enum UpdateMode : int { U_BATCH = 0, U_SINGLE = 1, U_FUSED = 2 };
+
+template <class R, int MODE>
+__global__ __launch_bounds__(NTH) void cg_update_kernel(CgArgs<R> A) {
+  __shared__ double sm[(NTH / 64) * 2];
+  __shared__ R win[VSUM_LDS_BYTES / sizeof(R)];
+  if constexpr (MODE == U_BATCH) {
+    __shared__ int list[NTH];
+    vertex_blocks(A.nvblk, true, list, [&](int vb) { return A.in[A.vblk_inst[vb]].act_eval != 0; }, [&](int vb) {
+      const InstState& st = A.in[A.vblk_inst[vb]];
+      cg_update_block<R, false>(A, vb, sm, win, (R)st.alpha, (R)st.pmean, st.cur);
+      __syncthreads();
+    });
+  } else {
+    __shared__ InstState st;
+    const int t = threadIdx.x;
+    if (t < STATE_DOUBLES) reinterpret_cast<double*>(&st)[t] = reinterpret_cast<const double*>(A.in)[t];
+    if constexpr (MODE == U_FUSED) {
+      __shared__ double red[SCAL_TH / 64];
+      const double dq = flat_sum_odd_short<SCAL_TH, NTH>(A.hq, A.nblocks, red);
+      if (t == 0) {
+        InstState s = st;
+        cg_alpha_step(s, dq);
+        st = s;
+      }
+    }
+    __syncthreads();
+    if (MODE == U_FUSED && blockIdx.x == 0 && t < STATE_DOUBLES)
+      reinterpret_cast<double*>(A.out)[t] = reinterpret_cast<double*>(&st)[t];
+    if (st.act_eval == 0) return;
+    for (int vb = blockIdx.x; vb < A.nvblk; vb += gridDim.x) {
+      cg_update_block<R, true>(A, vb, sm, win, (R)st.alpha, (R)st.pmean, st.cur);
+      __syncthreads();
+    }
+  }
 }
 
 }  // namespace apl
@@ -533,7 +624,7 @@ struct apl_solver {
   void* p = nullptr;       // PNCG direction: two buffers of V records of the mesh dtype
   void* g = nullptr;       // gradient: two buffers of V records, then the preconditioner (V records)
   void* cg = nullptr;      // CG: z (V records), d (two buffers of V records)
-  void* vecs = nullptr;    // CG: r, q, hd, t, b (N_VECS x V x 3)
+  void* vecs = nullptr;    // CG: r, hd, t, b (N_VECS x V x 3)
   uint32_t* own = nullptr;  // per slot: vertex and OWNER_BIT
   int32_t* iso = nullptr;  // vertices without tets, then their instances
   int n_iso = 0;
@@ -552,7 +643,7 @@ struct apl_solver {
 
 namespace apl {
 
-constexpr int N_VECS = 5;
+constexpr int N_VECS = 4;
 
 template <class R>
 static VecArgs<R> vec_args(apl_solver* s, const void* fext, const uint8_t* mask) {
@@ -628,7 +719,7 @@ static unsigned vec_grid(const apl_mesh* m) {
 }
 
 constexpr unsigned PASS_TRIAL = W_E | W_G | W_H | W_TRIAL, PASS_DIR = W_HQ | W_DIR;
-constexpr unsigned PASS_CGD = W_HP | W_CGD, PASS_ACT = W_HP | W_ACT;
+constexpr unsigned PASS_CGD = W_HP | W_VQ | W_CGD, PASS_ACT = W_HP | W_ACT;
 
 template <class R>
 static int pncg_iteration(apl_solver* s, const void* mu, const void* lam, const void* fext, const uint8_t* mask,
@@ -907,41 +998,63 @@ static CgArgs<R> cg_args(apl_solver* s, const void* rhs, void* y, const uint8_t*
   A.r = base;
   A.z = (Vec4<R>*)s->cg;
   A.d = (Vec4<R>*)s->cg + (size_t)m->L.V;
-  A.q = base + nv;
-  A.hd = base + 2 * nv;
-  A.t = base + 3 * nv;
+  A.hd = base + nv;
+  A.t = base + 2 * nv;
   A.tout = A.t;
+  A.nvblk = (int)m->L.vblk_inst.size();
+  A.nblocks = (int)m->L.nblocks;
   A.vblk_dots = m->d.vblk_dots;
-  A.st = s->st + m->L.n_inst;
+  A.t_dots = m->d.vblk_dots + 2 * (size_t)A.nvblk;
+  A.in = s->st + m->L.n_inst;
+  A.out = nullptr;
+  A.hq = s->hq;
   A.V = (size_t)m->L.V;
-  A.nvblk = (int)s->mesh->L.vblk_inst.size();
-  A.filter = s->mesh->L.n_inst > 1 ? 1 : 0;
   A.normal = 0;
   return A;
 }
 
 template <class R>
-static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const void* x, CgArgs<R>& A, double rtol,
+static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const void* x, CgArgs<R> A, double rtol,
                         int max_iters, hipStream_t st) {
   apl_mesh* m = s->mesh;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   const unsigned ni = (unsigned)m->L.n_inst;
+  InstState *sa = s->st, *sb = s->st + ni;  // after the beta step, after the alpha step
+  const bool single = ni == 1 && m->L.nblocks > 0;
   SolveArgs<R> S = solve_args<R>(s, true);
-  S.st = A.st;
-  if (launch_solve_pass<PASS_CGD, R>(m, s->material, mu, lam, x, nullptr, S, 0, st)) return -1;
+  S.prm.rtol = rtol;
+  S.prm.max_steps = max_iters;
+  int rc = 0;
+  if (single && nvb <= FUSE_CG_VBLOCKS) {
+    S.st = sb, S.out = sa;
+    S.table = m->d.vblk_dots, S.n_table = 2 * (int)nvb;
+    rc = launch_solve_pass<PASS_CGD | W_FUSED, R>(m, s->material, mu, lam, x, nullptr, S, 0, st);
+  } else {
+    hipLaunchKernelGGL(cg_beta_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sb, sa, rtol, max_iters, m->d.vblk_dots,
+                       m->d.inst_vblk_off);
+    S.st = sa;
+    rc = launch_solve_pass<PASS_CGD, R>(m, s->material, mu, lam, x, nullptr, S, 0, st);
+  }
+  if (rc) return -1;
   if (A.normal) {
-    // q = H (H d): t = H d with fixed DOFs zeroed, then the pass on t
-    CgArgs<R> At = A;
-    At.tout = A.t;
-    if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_T>), dim3(vec_grid(m)), dim3(NTH), 0, st, At);
+    // q = H (H d): t = H d with fixed DOFs zeroed, whose square is d.H^2 d, then the pass on t
+    A.in = sa;
+    if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_T>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+    S.st = sa;
     if (launch_solve_pass<PASS_ACT, R>(m, s->material, mu, lam, x, A.t, S, 0, st)) return -1;
   }
-  if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_Q>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, A.st, 2, rtol, max_iters, m->d.vblk_dots,
-                     m->d.inst_vblk_off);
-  if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_UPDATE>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, A.st, 3, rtol, max_iters, m->d.vblk_dots,
-                     m->d.inst_vblk_off);
+  if (single && !A.normal && m->L.nblocks <= FUSE_BLOCKS) {
+    A.in = sa, A.out = sb;
+    if (nvb) hipLaunchKernelGGL((cg_update_kernel<R, U_FUSED>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+  } else {
+    hipLaunchKernelGGL(cg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sa, sb, A.normal ? A.t_dots : s->hq,
+                       A.normal ? m->d.inst_vblk_off : m->d.inst_blk_off);
+    A.in = sb;
+    if (nvb && ni == 1)
+      hipLaunchKernelGGL((cg_update_kernel<R, U_SINGLE>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+    else if (nvb)
+      hipLaunchKernelGGL((cg_update_kernel<R, U_BATCH>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
+  }
   APL_CHECK_HIP(hipGetLastError());
   return 0;
 }
@@ -959,7 +1072,7 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
     // the normal equations' right-hand side H b (b with fixed DOFs zeroed),
     // kept by the solver; the CG then runs on it
     A.normal = 1;
-    R* b2 = (R*)s->vecs + 4 * 3 * (size_t)m->L.V;
+    R* b2 = (R*)s->vecs + 3 * 3 * (size_t)m->L.V;
     CgArgs<R> Ab = A;
     Ab.tout = A.t;
     if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_MASKCOPY>), dim3(vec_grid(m)), dim3(NTH), 0, st, Ab);
@@ -972,13 +1085,13 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   if (fill<R>(A.hd, 3 * (long long)m->L.V, R(0), st)) return -1;
   if (launch_elem(m, s->material, W_H, mu, lam, x, nullptr, nullptr, A.hd, 0, st)) return -1;
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_DIAG>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, A.st, 0, rtol, max_iters, m->d.vblk_dots,
-                     m->d.inst_vblk_off);
+  InstState* sb = s->st + n;
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, sb, 0, m->d.vblk_dots, m->d.inst_vblk_off);
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_PRECOND>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, A.st, 1, rtol, max_iters, m->d.vblk_dots,
-                     m->d.inst_vblk_off);
+  hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, sb, 1, m->d.vblk_dots, m->d.inst_vblk_off);
   APL_CHECK_HIP(hipGetLastError());
   solve_pass_grid<PASS_CGD, R>(m, s->material);
+  solve_pass_grid<PASS_CGD | W_FUSED, R>(m, s->material);
   if (normal) solve_pass_grid<PASS_ACT, R>(m, s->material);
   const int K = 16;
   // K iterations captured once per set of pointers and parameters
@@ -1020,6 +1133,8 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
       s->cg_gkey = key;
     }
   }
+  // (an update's residual is tested at the start of the next iteration, so an
+  // instance that ends with a launch's last update is seen to after the next launch)
   long long done = 0;
   while (true) {
     APL_CHECK_HIP(hipGraphLaunch(s->cg_gexec, st));

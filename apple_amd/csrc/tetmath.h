@@ -679,6 +679,7 @@ enum : unsigned {
   W_HQ = 16u,    // clamped quadratic form v^T H v
   W_MIX = 32u,   // mixed derivatives p^T dg/dmu, p^T dg/dlam (per tet)
   W_MIXA = 64u,  // mixed derivatives p^T dg/da_k, k = 0..5 (muscle activation, per tet)
+  W_VQ = 128u,   // v^T H v, unclamped (with W_HP)
 };
 
 template <class R>
@@ -688,6 +689,7 @@ struct TetOut {
   V3<R> h[4];   // max(dV diag H, 0)
   V3<R> hp[4];  // dV H v
   R hq;         // max(dV v^T H v, 0)
+  R vq;         // dV v^T H v
   R dmu, dlam;  // dV (dP/dmu):dF(v), dV (dP/dlam):dF(v)
   R dact[6];    // dV d(P:dF(v))/da_k (muscle)
 };
@@ -787,6 +789,7 @@ __host__ __device__ inline void tet_eval(const TetGeom<R>& g0, R mu, R lam, cons
 #pragma unroll
             for (int j = 0; j < 3; ++j) Tm.m[i][j] = lc * C.m[i][j] + muV * dF.m[i][j] + sV * Hs.m[i][j];
           if constexpr ((WHAT & W_HP) != 0) corner_products(Tm, g, o.hp);
+          if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot(Tm, dF);
         }
         if constexpr ((WHAT & W_MIX) != 0) {
           const M3<R> D = F_minus_cofF(G, I.trG);
@@ -854,6 +857,7 @@ __host__ __device__ inline void tet_eval(const TetGeom<R>& g0, R mu, R lam, cons
 #pragma unroll
           for (int j = 0; j < 3; ++j) T.m[i][j] = muV * (dF.m[i][j] - Qc.m[i][j]);
         corner_products(T, g, o.hp);
+        if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot(T, dF);
       }
       if constexpr ((WHAT & W_MIX) != 0) {
         o.dmu = g.dV * (S.sm1[0] * dM[0] + S.sm1[1] * dM[1] + S.sm1[2] * dM[2]);

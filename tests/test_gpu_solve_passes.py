@@ -56,6 +56,30 @@ def test_single_instance_equals_the_same_instance_of_a_batch(n):
         stb[0].n_steps, stb[0].n_evals, stb[0].f, stb[0].grad_norm, stb[0].alpha, stb[0].beta)
 
 
+# likewise the CG: the step from the blocks' d.Hd (2,048 element blocks), beta
+# from two columns per vertex block (1,024 of them), and the normal equations
+@pytest.mark.parametrize("n,normal", [(2, False), (46, False), (47, False), (63, False), (64, False), (6, True)])
+def test_single_cg_equals_the_same_instance_of_a_batch(n, normal):
+    print(f"[passes] CG n = {n} normal {normal}", flush=True)
+    m, fixed, x0, f = _case(n)
+    m2, fixed2, x2, f2 = _case(3, seed=1)
+    r, r2 = Region.from_mesh(m), Region.from_mesh(m2)
+    pot = fem.StableNeoHookean.from_region(r, device="cuda")
+    t = lambda a: torch.as_tensor(a, dtype=torch.float32, device="cuda").contiguous()  # noqa: E731
+    rhs, rhs2 = t(np.random.default_rng(4).standard_normal(x0.shape)), t(np.random.default_rng(5).standard_normal(x2.shape))
+    kw = dict(rtol=1e-12, max_iters=7, normal=normal)
+    y = torch.empty_like(rhs)
+    st = DeviceSolver(pot).cg(t(0.1 * x0), rhs, y, mask_bits(fixed, "cuda"), **kw)[0]
+    b = batch.Batch([batch.Instance(r2, m2.cell_data["mu"], m2.cell_data["lambda"], f2, fixed2, x2),
+                     batch.Instance(r, m.cell_data["mu"], m.cell_data["lambda"], f, fixed, x0)], _lib.APL_SNH, device="cuda")
+    yb = torch.empty_like(b.x0)
+    stb = b.solver().cg(t(torch.cat([t(0.1 * x2), t(0.1 * x0)])), torch.cat([rhs2, rhs]), yb, b.mask, **kw)[1]
+    assert st.n_steps == 7 and torch.isfinite(y).all()
+    assert torch.equal(b.split(yb)[1], y)
+    assert (st.result, st.n_steps, st.f, st.grad_norm, st.alpha, st.beta) == (
+        stb.result, stb.n_steps, stb.f, stb.grad_norm, stb.alpha, stb.beta)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("cls", [fem.StableNeoHookean, fem.Arap])
 def test_vertices_without_tets(cls, dtype):
