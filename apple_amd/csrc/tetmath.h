@@ -277,12 +277,14 @@ __host__ __device__ inline float fast_rsq(float x) {
 #endif
 }
 
-// 1/x and 1/sqrt(x): the hardware approximations (about 1 ulp) in FP32,
+// 1/x, 1/sqrt(x), sqrt(x): the hardware approximations (about 1 ulp) in FP32,
 // correctly rounded division and square root in FP64
 __host__ __device__ inline float recip(float x) { return fast_rcp(x); }
 __host__ __device__ inline double recip(double x) { return 1.0 / x; }
 __host__ __device__ inline float rsqrt_r(float x) { return fast_rsq(x); }
 __host__ __device__ inline double rsqrt_r(double x) { return 1.0 / sqrt(x); }
+__host__ __device__ inline float sqrt_r(float x) { return fast_sqrt(x); }
+__host__ __device__ inline double sqrt_r(double x) { return sqrt(x); }
 
 __host__ __device__ inline void jacobi_rotate_fast(float (&a)[3][3], M3<float>& V, int p, int q) {
   const float apq = a[p][q];
@@ -328,7 +330,7 @@ __host__ __device__ inline void swap_cols(M3<R>& V, R (&e)[3], int i, int j) {
 template <class R>
 __host__ __device__ inline void sigma_from(R e, R q, R& s, R& sm1) {
   if (fabs(e) < R(0.25) && q > R(0)) {
-    sm1 = e * recip(R(1) + sqrt(R(1) + e));
+    sm1 = e * recip(R(1) + sqrt_r(R(1) + e));
     s = R(1) + sm1;
   } else {
     s = q;
@@ -377,20 +379,15 @@ __host__ __device__ inline void sort_eig(const R (&a)[3][3], M3<R>& V, R (&e)[3]
   if (e[1] < e[2]) swap_cols(V, e, 1, 2);
 }
 
-// U and sigma from the sorted eigenpairs (e, V) of F^T F - I.
+// U, sigma and sigma - 1 from the sorted eigenpairs of F^T F - I: v0 the first
+// eigenvector, f0, f1, f2 the columns of F V, e the eigenvalues.  u: U's columns.
 template <class R>
-__host__ __device__ inline Svd<R> qr_sigma(const M3<R>& G, const M3<R>& V0, const R (&e)[3]) {
-  Svd<R> r;
-  M3<R>& V = r.V;
-  V = V0;
+__host__ __device__ inline void qr_sigma(V3<R> v0, V3<R> f0, V3<R> f1, V3<R> f2, const R (&e)[3], V3<R> (&u)[3],
+                                         R (&s)[3], R (&sm1)[3]) {
   // U and the singular values by Gram-Schmidt QR of F V, F = I + G
   // (the QR step of McAdams et al., "Computing the SVD of 3x3 matrices with
   // minimal branching", 2011): sigma = diag(R) keeps absolute accuracy
   // eps*|F| even for near-singular F, unlike sqrt(1 + e_i).
-  V3<R> v0 = col(V, 0), v1 = col(V, 1), v2 = col(V, 2);
-  V3<R> f0 = v0 + mul(G, v0);
-  V3<R> f1 = v1 + mul(G, v1);
-  V3<R> f2 = v2 + mul(G, v2);
   // squared-norm floors: normal numbers in either precision
   const R tiny = sizeof(R) == 4 ? R(1e-36) : R(1e-60);
   const R d0 = dot(f0, f0);
@@ -416,12 +413,23 @@ __host__ __device__ inline Svd<R> qr_sigma(const M3<R>& G, const M3<R>& V0, cons
     u1 = rsqrt_r(dot(w, w)) * w;
   }
   V3<R> u2 = cross(u0, u1);
-  set_col(r.U, 0, u0);
-  set_col(r.U, 1, u1);
-  set_col(r.U, 2, u2);
-  sigma_from(e[0], n0, r.s[0], r.sm1[0]);
-  sigma_from(e[1], n1, r.s[1], r.sm1[1]);
-  sigma_from(e[2], dot(u2, f2), r.s[2], r.sm1[2]);
+  u[0] = u0;
+  u[1] = u1;
+  u[2] = u2;
+  sigma_from(e[0], n0, s[0], sm1[0]);
+  sigma_from(e[1], n1, s[1], sm1[1]);
+  sigma_from(e[2], dot(u2, f2), s[2], sm1[2]);
+}
+
+template <class R>
+__host__ __device__ inline Svd<R> qr_sigma(const M3<R>& G, const M3<R>& V, const R (&e)[3]) {
+  Svd<R> r;
+  r.V = V;
+  const V3<R> v0 = col(V, 0), v1 = col(V, 1), v2 = col(V, 2);
+  V3<R> u[3];
+  qr_sigma(v0, v0 + mul(G, v0), v1 + mul(G, v1), v2 + mul(G, v2), e, u, r.s, r.sm1);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) set_col(r.U, k, u[k]);
   return r;
 }
 
@@ -453,51 +461,86 @@ __host__ __device__ inline Svd<R> svd_rv(const M3<R>& G) {
 #ifndef REFINE_F64_SWEEPS
 #define REFINE_F64_SWEEPS 1
 #endif
+// One FP64 Jacobi rotation of b = f^T f - I in the plane (p, q), applied to
+// the basis v and to f = F v.
+__host__ __device__ inline void jacobi_rotate_vf(double (&b)[3][3], V3<double> (&v)[3], V3<double> (&f)[3], int p,
+                                                 int q) {
+  const double bpq = b[p][q];
+  const double scale = fabs(b[p][p]) + fabs(b[q][q]);
+  if (!(fabs(bpq) > 1e-30 + scale * 1e-18)) return;
+  const double tau = (b[q][q] - b[p][p]) / (2.0 * bpq);
+  const double t = (tau >= 0.0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+  const double c = 1.0 / sqrt(1.0 + t * t), s = t * c;
+  b[p][p] -= t * bpq;
+  b[q][q] += t * bpq;
+  b[p][q] = b[q][p] = 0.0;
+  const int r = 3 - p - q;
+  const double brp = b[r][p], brq = b[r][q];
+  b[r][p] = b[p][r] = c * brp - s * brq;
+  b[r][q] = b[q][r] = s * brp + c * brq;
+  const V3<double> vp = v[p], fp = f[p];
+  v[p] = c * vp - s * v[q];
+  v[q] = s * vp + c * v[q];
+  f[p] = c * fp - s * f[q];
+  f[q] = s * fp + c * f[q];
+}
+__host__ __device__ inline void swap_vf(V3<double> (&v)[3], V3<double> (&f)[3], double (&e)[3], int i, int j) {
+  if (!(e[i] < e[j])) return;
+  const double t = e[i];
+  e[i] = e[j];
+  e[j] = t;
+  const V3<double> a = v[i], g = f[i];
+  v[i] = v[j];
+  v[j] = -1.0 * a;  // keep det V = +1
+  f[i] = f[j];
+  f[j] = -1.0 * g;
+}
+
 // FP64 finish from an FP32 eigenbasis Vf of F^T F - I: re-orthonormalise
-// Vf in FP64, rotate the FP64 F^T F - I into it (nearly diagonal), one FP64
-// sweep, then the FP64 sort and QR; results rounded to R.
+// Vf in FP64, one FP64 sweep on b = (F V)^T (F V) - I (nearly diagonal; in
+// FP64 the subtraction costs 1e-16 absolute), whose rotations go to V and to
+// F V, then the FP64 sort and QR; results rounded to R.  Keeping F V instead
+// of forming F^T F - I and rotating it leaves the kernels' registers to the
+// rest of the element (the FP64 matrices set their peak).
 template <class R>
 __host__ __device__ inline Svd<R> svd_finish_f64(const M3<R>& G, const M3<float>& Vf) {
-  M3<double> Gd;
+  V3<double> v[3], f[3];
+  v[0] = v3((double)Vf.m[0][0], (double)Vf.m[1][0], (double)Vf.m[2][0]);
+  v[1] = v3((double)Vf.m[0][1], (double)Vf.m[1][1], (double)Vf.m[2][1]);
+  v[0] = (1.0 / sqrt(dot(v[0], v[0]))) * v[0];
+  v[1] = v[1] - dot(v[0], v[1]) * v[0];
+  v[1] = (1.0 / sqrt(dot(v[1], v[1]))) * v[1];
+  v[2] = cross(v[0], v[1]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    f[k] = v[k] + v3((double)G.m[0][0] * v[k].x + (double)G.m[0][1] * v[k].y + (double)G.m[0][2] * v[k].z,
+                     (double)G.m[1][0] * v[k].x + (double)G.m[1][1] * v[k].y + (double)G.m[1][2] * v[k].z,
+                     (double)G.m[2][0] * v[k].x + (double)G.m[2][1] * v[k].y + (double)G.m[2][2] * v[k].z);
+  double b[3][3];
 #pragma unroll
   for (int i = 0; i < 3; ++i)
 #pragma unroll
-    for (int j = 0; j < 3; ++j) Gd.m[i][j] = (double)G.m[i][j];
-  double ad[3][3], t[3][3], b[3][3];
-  ftf_minus_i(Gd, ad);
-  V3<double> c0 = v3((double)Vf.m[0][0], (double)Vf.m[1][0], (double)Vf.m[2][0]);
-  V3<double> c1 = v3((double)Vf.m[0][1], (double)Vf.m[1][1], (double)Vf.m[2][1]);
-  c0 = (1.0 / sqrt(dot(c0, c0))) * c0;
-  c1 = c1 - dot(c0, c1) * c0;
-  c1 = (1.0 / sqrt(dot(c1, c1))) * c1;
-  const V3<double> c2 = cross(c0, c1);
-  M3<double> V;
-  set_col(V, 0, c0);
-  set_col(V, 1, c1);
-  set_col(V, 2, c2);
-  // b = V^T ad V
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) t[i][j] = ad[i][0] * V.m[0][j] + ad[i][1] * V.m[1][j] + ad[i][2] * V.m[2][j];
-#pragma unroll
-  for (int i = 0; i < 3; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) b[i][j] = V.m[0][i] * t[0][j] + V.m[1][i] * t[1][j] + V.m[2][i] * t[2][j];
-  jacobi_sweeps(b, V, REFINE_F64_SWEEPS);
-  double ed[3];
-  sort_eig(b, V, ed);
-  const Svd<double> Sd = qr_sigma(Gd, V, ed);
+    for (int j = i; j < 3; ++j) b[i][j] = b[j][i] = dot(f[i], f[j]) - (i == j ? 1.0 : 0.0);
+  for (int sw = 0; sw < REFINE_F64_SWEEPS; ++sw) {
+    jacobi_rotate_vf(b, v, f, 0, 1);
+    jacobi_rotate_vf(b, v, f, 0, 2);
+    jacobi_rotate_vf(b, v, f, 1, 2);
+  }
+  double e[3] = {b[0][0], b[1][1], b[2][2]};
+  swap_vf(v, f, e, 0, 1);
+  swap_vf(v, f, e, 0, 2);
+  swap_vf(v, f, e, 1, 2);
   Svd<R> S;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    S.s[i] = (R)Sd.s[i];
-    S.sm1[i] = (R)Sd.sm1[i];
+  for (int k = 0; k < 3; ++k) set_col(S.V, k, v3((R)v[k].x, (R)v[k].y, (R)v[k].z));
+  V3<double> u[3];
+  double sg[3], sm1[3];
+  qr_sigma(v[0], f[0], f[1], f[2], e, u, sg, sm1);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      S.U.m[i][j] = (R)Sd.U.m[i][j];
-      S.V.m[i][j] = (R)Sd.V.m[i][j];
-    }
+  for (int k = 0; k < 3; ++k) {
+    S.s[k] = (R)sg[k];
+    S.sm1[k] = (R)sm1[k];
+    set_col(S.U, k, v3((R)u[k].x, (R)u[k].y, (R)u[k].z));
   }
   return S;
 }
@@ -527,12 +570,11 @@ __host__ __device__ inline Svd<R> svd_rv_refined(const M3<R>& G) {
 // The same SVD with FP32 arithmetic except one step: F^T F - I is formed
 // in FP64 from the FP32 G (exact products, one rounding to FP32), which
 // removes the cancellation that G + G^T + G^T G suffers in FP32 under a
-// large rotation (|G| ~ 1 while the strain is small).  Then FP32 Jacobi
-// sweeps with hardware-approximate rotations, the FP32 QR of F V for U and
-// the FP32 singular values (sigma - 1 from the eigenvalue near 1).  The
-// stress mu U diag(sigma - 1) V^T and the twist-mode projection are smooth
-// functions of F^T F, so the eigenvectors' FP32 error within nearly
-// degenerate pairs does not reach them.
+// large rotation (|G| ~ 1 while the strain is small).  Then the closed-form
+// FP32 eigenvectors, the FP32 QR of F V for U and the FP32 singular values
+// (sigma - 1 from the eigenvalue near 1).  The stress mu U diag(sigma - 1) V^T
+// and the twist-mode projection are smooth functions of F^T F, so the
+// eigenvectors' FP32 error within nearly degenerate pairs does not reach them.
 #ifndef E32_SWEEPS
 #define E32_SWEEPS 4
 #endif
@@ -561,28 +603,102 @@ __host__ __device__ inline void jacobi_fast_sweeps(float (&a)[3][3], M3<float>& 
   }
 }
 
-// The ARAP kernels' SVD.  Every element gets the FP32 basis (F^T F - I
-// formed in FP64, FP32 Jacobi sweeps); elements with det F > 1/64 (large
-// rotations and large strains included) finish in FP32 (sort, QR), the
-// inverted and nearly flat ones in FP64 from that basis (svd_finish_f64):
-// there the rotation-variant sign convention hinges on the sign of det F and
-// on comparisons of nearly equal |sigma| that FP32 can get the other way.
-// The threshold keeps the FP32 det3's rounding (~1e-7 |F|^3) far from
-// deciding the branch; only the finish is divergent within a wave.
+// Eigenvalues e (descending) and eigenvectors V (a rotation) of a symmetric a,
+// in closed form.  With B the traceless part of a over its norm, the
+// eigenvalues of B are 2 cos(theta + 2 k pi / 3), cos 3 theta = det B / 2
+// (the trigonometric solution of the depressed cubic): the one farthest from
+// the others is beta = 2 cos(acos(|h|) / 3) in [sqrt 3, 2] with the sign of
+// h = det B / 2, a smooth function of |h| (here a cubic and one Newton step,
+// 4e-9 off).  It is at least sqrt 3 away from the others, so the columns of
+// the cofactors of B - beta I give its vector to a few ulp however close
+// those two are; the plane orthogonal to it (orthonormal basis after Duff et
+// al., "Building an Orthonormal Basis, Revisited", JCGT 2017) is left with a
+// 2x2 problem, one exact rotation.
+// Against four cyclic Jacobi sweeps the ARAP pass issues 979 instead of 1,350
+// VALU instructions per 64 tets; the 64^3 pass went from 64.4 to 53.9 us and
+// its error against 64 bits from 2.8e-7 to 2.3e-7.
+__host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, float (&e)[3]) {
+  const float q = (a[0][0] + a[1][1] + a[2][2]) * (1.0f / 3.0f);
+  float b00 = a[0][0] - q, b11 = a[1][1] - q, b22 = a[2][2] - q;
+  float b01 = a[0][1], b02 = a[0][2], b12 = a[1][2];
+  // scaled by the largest entry first: no square over- or underflows
+  const float m = fmaxf(fmaxf(fmaxf(fabsf(b00), fabsf(b11)), fmaxf(fabsf(b22), fabsf(b01))),
+                        fmaxf(fabsf(b02), fabsf(b12)));
+  const float im = m > 1e-30f ? fast_rcp(m) : 0.0f;
+  b00 *= im, b11 *= im, b22 *= im, b01 *= im, b02 *= im, b12 *= im;
+  const float p2 = (b00 * b00 + b11 * b11 + b22 * b22) * (1.0f / 6.0f) + (b01 * b01 + b02 * b02 + b12 * b12) * (1.0f / 3.0f);
+  const float ip = p2 > 0.0f ? fast_rsq(p2) : 0.0f;
+  const float scale = m * (p2 * ip);
+  b00 *= ip, b11 *= ip, b22 *= ip, b01 *= ip, b02 *= ip, b12 *= ip;
+  const float h = 0.5f * (b00 * (b11 * b22 - b12 * b12) - b01 * (b01 * b22 - b12 * b02) + b02 * (b01 * b12 - b11 * b02));
+  const float ah = fabsf(h);
+  float beta = 1.73211585f + ah * (0.33095008f + ah * (-0.08213921f + ah * 0.01913826f));
+  const float bb = beta * beta;
+  beta -= (beta * (bb - 3.0f) - 2.0f * ah) * fast_rcp(3.0f * bb - 3.0f);
+  const bool top = h >= 0.0f;
+  const float l = top ? beta : -beta;
+  // cofactors of B - l I; the column of the largest diagonal entry
+  const float c00 = b00 - l, c11 = b11 - l, c22 = b22 - l;
+  const float k00 = c11 * c22 - b12 * b12, k11 = c00 * c22 - b02 * b02, k22 = c00 * c11 - b01 * b01;
+  const float k01 = b02 * b12 - b01 * c22, k02 = b01 * b12 - b02 * c11, k12 = b01 * b02 - b12 * c00;
+  const bool s1 = k11 > k00;
+  const float kd = s1 ? k11 : k00;
+  const bool s2 = k22 > kd;
+  V3<float> v = v3(s2 ? k02 : (s1 ? k01 : k00), s2 ? k12 : (s1 ? k11 : k01), s2 ? k22 : (s1 ? k12 : k02));
+  v = fast_rsq(dot(v, v)) * v;
+  const float sg = v.z >= 0.0f ? 1.0f : -1.0f;
+  const float w = -fast_rcp(sg + v.z), xy = v.x * v.y * w;
+  V3<float> x = v3(1.0f + sg * v.x * v.x * w, sg * xy, -sg * v.x);
+  V3<float> y = v3(xy, sg + v.y * v.y * w, -v.y);  // x cross y = v
+  const V3<float> bx = v3(b00 * x.x + b01 * x.y + b02 * x.z, b01 * x.x + b11 * x.y + b12 * x.z,
+                          b02 * x.x + b12 * x.y + b22 * x.z);
+  const V3<float> by = v3(b00 * y.x + b01 * y.y + b02 * y.z, b01 * y.x + b11 * y.y + b12 * y.z,
+                          b02 * y.x + b12 * y.y + b22 * y.z);
+  const float m00 = dot(x, bx), m11 = dot(y, by), m01 = dot(x, by);
+  // rotation by the smaller angle, the larger eigenvalue first
+  const float d = 0.5f * (m00 - m11), den = fabsf(d) + fast_sqrt(d * d + m01 * m01);
+  const float t = den > 0.0f ? m01 * fast_rcp(den) : 0.0f;  // tan of the angle, up to the sign of d
+  const float c = fast_rsq(1.0f + t * t), s = t * c;
+  const bool sw = d < 0.0f;
+  // d >= 0: v1 = c x + s y, v2 = c y - s x; d < 0: v1 = s x + c y, v2 = s y - c x
+  const float ca = sw ? s : c, sa = sw ? c : s;
+  const V3<float> v1 = ca * x + sa * y, v2 = ca * y - sa * x;
+  const float big = (sw ? m11 : m00) + t * m01, small = (sw ? m00 : m11) - t * m01;
+  const float e1 = q + scale * big, e2 = q + scale * small, el = q + scale * l;
+  e[0] = top ? el : e1;
+  e[1] = top ? e1 : e2;
+  e[2] = top ? e2 : el;
+  set_col(V, 0, v3(top ? v.x : v1.x, top ? v.y : v1.y, top ? v.z : v1.z));
+  set_col(V, 1, v3(top ? v1.x : v2.x, top ? v1.y : v2.y, top ? v1.z : v2.z));
+  set_col(V, 2, v3(top ? v2.x : v.x, top ? v2.y : v.y, top ? v2.z : v.z));
+}
+
+// The ARAP kernels' SVD: F^T F - I formed in FP64, then elements with
+// det F > 1/64 and det F > |F|^3 / 362 (large rotations and large strains
+// included) finish in FP32 (closed-form eigenvectors, QR), the inverted and
+// nearly flat ones in FP64 from the FP32 Jacobi basis (svd_finish_f64): there
+// the rotation-variant sign convention hinges on the sign of det F and on
+// comparisons of nearly equal |sigma| that FP32 can get the other way, and
+// the Jacobi basis keeps an already diagonal F^T F as it is, ties included.
+// The first threshold keeps the FP32 det3's rounding (~1e-7 |F|^3) far from
+// deciding the branch; the second is met by elements drawn out more than
+// about 10:1, where the rotation about the long axis amplifies FP32 rounding
+// by sigma_0 / (sigma_1 + sigma_2).  Only those elements' branch is divergent.
 __host__ __device__ inline Svd<float> svd_rv_fast(const M3<float>& G) {
   float a[3][3];
   ftf_minus_i_f64(G, a);
   M3<float> V;
-  jacobi_fast_sweeps(a, V);
   M3<float> F = G;
   F.m[0][0] += 1.0f;
   F.m[1][1] += 1.0f;
   F.m[2][2] += 1.0f;
-  if (det3(F) > 0.015625f) {
+  const float det = det3(F), f2 = 3.0f + (a[0][0] + a[1][1] + a[2][2]);
+  if (det > 0.015625f && det * det * 131072.0f > f2 * f2 * f2) {
     float e[3];
-    sort_eig(a, V, e);
+    eig_sym3(a, V, e);
     return qr_sigma(G, V, e);
   }
+  jacobi_fast_sweeps(a, V);
   return svd_finish_f64(G, V);
 }
 
@@ -616,18 +732,17 @@ __host__ __device__ inline void arap_lambdas(const R s[3], R lam[3]) {
   lam[2] = R(2) * recip(p2 > R(2) ? p2 : R(2));
 }
 
-// Twist-mode coordinates of a vector d: (Q0 d, Q1 d, Q2 d) (func/_misc.py:56-70)
+// Twist-mode coordinates of a vector d times sqrt 2: sqrt 2 (Q0 d, Q1 d, Q2 d) (func/_misc.py:56-70)
 //   Q0 = (U1 V0^T - U0 V1^T)/sqrt2, Q1 = (U1 V2^T - U2 V1^T)/sqrt2, Q2 = (U0 V2^T - U2 V0^T)/sqrt2
 template <class R>
 __host__ __device__ inline void twist_apply(const Svd<R>& S, V3<R> d, V3<R> out[3]) {
-  const R r2 = R(0.70710678118654752440);
   R w0 = S.V.m[0][0] * d.x + S.V.m[1][0] * d.y + S.V.m[2][0] * d.z;
   R w1 = S.V.m[0][1] * d.x + S.V.m[1][1] * d.y + S.V.m[2][1] * d.z;
   R w2 = S.V.m[0][2] * d.x + S.V.m[1][2] * d.y + S.V.m[2][2] * d.z;
   V3<R> U0 = col(S.U, 0), U1 = col(S.U, 1), U2 = col(S.U, 2);
-  out[0] = r2 * (w0 * U1 - w1 * U0);
-  out[1] = r2 * (w2 * U1 - w1 * U2);
-  out[2] = r2 * (w2 * U0 - w0 * U2);
+  out[0] = w0 * U1 - w1 * U0;
+  out[1] = w2 * U1 - w1 * U2;
+  out[2] = w2 * U0 - w0 * U2;
 }
 
 // Q_k : dF for k = 0,1,2 via M = U^T dF V
@@ -830,14 +945,25 @@ __host__ __device__ inline void tet_eval(const TetGeom<R>& g0, R mu, R lam, cons
     R lk[3];
     if constexpr ((WHAT & (W_H | W_HP | W_HQ)) != 0) arap_lambdas(S.s, lk);
     if constexpr ((WHAT & W_H) != 0) {
+      // corner 0 last: its mode coordinates are minus the sum of the others'
+      const R hl[3] = {R(0.5) * lk[0], R(0.5) * lk[1], R(0.5) * lk[2]};
+      V3<R> q0[3] = {v3(R(0), R(0), R(0)), v3(R(0), R(0), R(0)), v3(R(0), R(0), R(0))};
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
+      for (int aa = 1; aa <= 4; ++aa) {
+        const int a = aa & 3;
         V3<R> qd[3];
-        twist_apply(S, g.d[a], qd);
+        if (a != 0) {
+          twist_apply(S, g.d[a], qd);
+#pragma unroll
+          for (int k = 0; k < 3; ++k) q0[k] = q0[k] + qd[k];
+        } else {
+#pragma unroll
+          for (int k = 0; k < 3; ++k) qd[k] = q0[k];  // (only squared)
+        }
         R t = dot(g.d[a], g.d[a]);
-        R hx = muV * (t - (lk[0] * qd[0].x * qd[0].x + lk[1] * qd[1].x * qd[1].x + lk[2] * qd[2].x * qd[2].x));
-        R hy = muV * (t - (lk[0] * qd[0].y * qd[0].y + lk[1] * qd[1].y * qd[1].y + lk[2] * qd[2].y * qd[2].y));
-        R hz = muV * (t - (lk[0] * qd[0].z * qd[0].z + lk[1] * qd[1].z * qd[1].z + lk[2] * qd[2].z * qd[2].z));
+        R hx = muV * (t - (hl[0] * qd[0].x * qd[0].x + hl[1] * qd[1].x * qd[1].x + hl[2] * qd[2].x * qd[2].x));
+        R hy = muV * (t - (hl[0] * qd[0].y * qd[0].y + hl[1] * qd[1].y * qd[1].y + hl[2] * qd[2].y * qd[2].y));
+        R hz = muV * (t - (hl[0] * qd[0].z * qd[0].z + hl[1] * qd[1].z * qd[1].z + hl[2] * qd[2].z * qd[2].z));
         o.h[a] = v3(hx > R(0) ? hx : R(0), hy > R(0) ? hy : R(0), hz > R(0) ? hz : R(0));
       }
     }
