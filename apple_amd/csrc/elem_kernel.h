@@ -443,6 +443,14 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   const int n_cand = k0 < nb_x ? (nb_x - k0 + K - 1) / K : 0;
   bool filter = false;
   InstScalars single;  // the instance's scalars (FUSED)
+  // the vertex of slot s of the block whose slots start at sb (with OWNER_BIT
+  // where the pass needs it)
+  auto slot_vertex = [&](int sb, int s) -> uint32_t {
+    if constexpr (DIR || CGD)
+      return at(S.own + sb, (unsigned)s);
+    else
+      return (uint32_t)at(A.loc_gid + sb, (unsigned)s);
+  };
   // FUSED: the first block's tables, records and slot vertices are loaded
   // before the scalar step, whose sums and barriers hide their latency
   int pre_b = -1;
@@ -451,10 +459,10 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   if constexpr (FUSED) {
     if (n_cand > 0) {
       pre_b = xcd_block(k0);
-      const int t0 = A.blk_tet_off[pre_b], sb = A.blk_loc_off[pre_b];
-      if (tid < A.blk_tet_off[pre_b + 1] - t0) load_rec<MAT>(block_res<MAT>(A, t0), (unsigned)tid, pre_rec);
-      if (tid < A.blk_loc_off[pre_b + 1] - sb)
-        pre_o = TRIAL ? (uint32_t)at(A.loc_gid + sb, (unsigned)tid) : at(S.own + sb, (unsigned)tid);
+      const int t0 = A.blk_tet_off[pre_b], t1 = A.blk_tet_off[pre_b + 1];
+      const int sb = A.blk_loc_off[pre_b], sb1 = A.blk_loc_off[pre_b + 1];
+      pre_o = slot_vertex(sb, min(tid, sb1 - sb - 1));
+      load_rec<MAT>(block_res<MAT>(A, t0), (unsigned)min(tid, t1 - t0 - 1), pre_rec);
     }
     scalar_step<WHAT>(S, st_lds, smem_d + HEAD);
     if constexpr (DIR) step_isolated(S, st_lds);
@@ -497,71 +505,88 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         else
           return S;
       }();
-      const int t0 = A.blk_tet_off[b];
-      const int nt = A.blk_tet_off[b + 1] - t0;
-      const int sb = A.blk_loc_off[b];
-      const int nloc = A.blk_loc_off[b + 1] - sb;
+      // Everything a block reads that does not depend on another load of it is
+      // started here, without a branch between: the tables by scalar loads, then
+      // the thread's slot vertex, its tet record and the destinations of its
+      // slot partials (idle threads read the block's last entries), so the
+      // staging waits for the slot vertex alone.  With the destinations first
+      // and each load under its own branch a block took five memory latencies
+      // in turn, now three: 51^3 H v 27.6 -> 25.9 us, FP64 pass at 37^3 25.9 ->
+      // 24.4 us, 64^3 solve 55.6 -> 53.1 ms.
+      const int t0 = A.blk_tet_off[b], t1 = A.blk_tet_off[b + 1];
+      const int sb = A.blk_loc_off[b], sb1 = A.blk_loc_off[b + 1];
+      const int nt = t1 - t0, nloc = sb1 - sb;
       const int lg = (4 * nloc <= SPT * NTH) ? 2 : ((2 * nloc <= SPT * NTH) ? 1 : 0);
       const int tps = 1 << lg;
-      // destinations of this thread's slot partials, loaded early
+      const BlockRes br = block_res<MAT>(A, t0);
+      uint32_t o0 = pre_o;
+      TetRec<R> rec;
+      if (FUSED && b == pre_b) {
+        rec = pre_rec;
+      } else {
+        o0 = slot_vertex(sb, min(tid, nloc - 1));
+        __builtin_amdgcn_sched_barrier(0);  // this load first: the staging waits for it alone
+        load_rec<MAT>(br, (unsigned)min(tid, nt - 1), rec);
+      }
       int dst_pre[SPT];
       if constexpr (SCATTER) {
 #pragma unroll
-        for (int k = 0; k < SPT; ++k) {
-          const int item = tid + k * NTH;
-          const int s = item >> lg;
-          dst_pre[k] = (s < nloc && (item & (tps - 1)) == 0) ? at(A.loc_dst + sb, (unsigned)s) : 0;
-        }
+        for (int k = 0; k < SPT; ++k)
+          dst_pre[k] = at(A.loc_dst + sb, (unsigned)min((tid + k * NTH) >> lg, nloc - 1));
       }
-
-      // this thread's first tet record, loaded before the staging barrier so the
-      // two global-load latencies overlap
-      const BlockRes br = block_res<MAT>(A, t0);
-      TetRec<R> rec;
-      if (FUSED && b == pre_b)
-        rec = pre_rec;
-      else if (tid < nt)
-        load_rec<MAT>(br, (unsigned)tid, rec);
+      // (a vertex is never all ones; asked here, or the compiler moves the load of
+      // o0 down into the staging's branch, behind the others)
+      const int s_first = o0 != ~0u ? tid : nloc;
 
       // stage the block's vertex window (u = x + alpha p for a trial point; the
-      // new iterate and direction for an accepted step)
-      const int32_t* gids = A.loc_gid + sb;
+      // new iterate and direction for an accepted step): stage(slot, o), o its
+      // vertex as slot_vertex gives it
+      auto put_u = [&](int s, const Vec4<X>& u4) { *reinterpret_cast<Vec4<X>*>(u_lds + 4 * s) = u4; };
+      auto put_v = [&](int s, const Vec4<R>& v4) { *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4; };
+      auto window = [&](auto stage) {
+        // the thread's first slot apart from the others, or the wait at the
+        // loop's head would be for the tet records too; and a vertex is never
+        // all ones: asked here, so that the load of o0 is not moved down into
+        // this branch, behind the others
+        if (tid < nloc && o0 != ~0u) {
+          stage(tid, o0);
+          for (int s = tid + NTH; s < nloc; s += NTH) stage(s, slot_vertex(sb, s));
+        }
+      };
       if constexpr (DIR) {
         const Step<R> step(S, st);
-        for (int s = tid; s < nloc; s += NTH) {
-          const uint32_t o = FUSED && b == pre_b && s == tid ? pre_o : at(S.own + sb, (unsigned)s);
+        window([&](int s, uint32_t o) {
           Vec4<X> u4;
           Vec4<R> v4;
           step_vertex(step, o & ~OWNER_BIT, (o & OWNER_BIT) != 0, u4, v4);
-          *reinterpret_cast<Vec4<X>*>(u_lds + 4 * s) = u4;
-          *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4;
-        }
+          put_u(s, u4);
+          put_v(s, v4);
+        });
         if (!step.dir) return;  // converged at this step: no new direction
       } else if constexpr (CGD) {
         const Direction<R> dir(S, st);
-        for (int s = tid; s < nloc; s += NTH) {
-          const uint32_t o = at(S.own + sb, (unsigned)s);
+        window([&](int s, uint32_t o) {
           const unsigned v = o & ~OWNER_BIT;
-          Vec4<X> u4 = {{at(A.x, 3u * v), at(A.x, 3u * v + 1), at(A.x, 3u * v + 2), X(0)}};
+          const Vec4<X> u4 = {{at(A.x, 3u * v), at(A.x, 3u * v + 1), at(A.x, 3u * v + 2), X(0)}};
           Vec4<R> v4;
           direction_vertex(dir, v, (o & OWNER_BIT) != 0, v4);
-          *reinterpret_cast<Vec4<X>*>(u_lds + 4 * s) = u4;
-          *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4;
-        }
+          put_u(s, u4);
+          put_v(s, v4);
+        });
       } else if constexpr (TRIAL) {
         const double alpha = st.alpha;
         const Vec4<double>* xb = S.x + (st.cur ? S.V : (size_t)0);
         const Vec4<R>* pb = S.p + (st.cur ? S.V : (size_t)0);
-        for (int s = tid; s < nloc; s += NTH) {
-          const size_t v = FUSED && b == pre_b && s == tid ? (size_t)pre_o : (size_t)at(gids, (unsigned)s);
+        window([&](int s, uint32_t o) {
+          const size_t v = o;
           Vec4<double> u4 = xb[v];
           const Vec4<R> p4 = pb[v];
 #pragma unroll
           for (int c = 0; c < 3; ++c) u4.v[c] += alpha * (double)p4.v[c];
-          *reinterpret_cast<Vec4<X>*>(u_lds + 4 * s) = u4;
-        }
+          put_u(s, u4);
+        });
       } else {
-        for (int s = tid; s < nloc; s += NTH) {
+        window([&](int s, uint32_t o) {
           X ux, uy, uz;
           R px = R(0), py = R(0), pz = R(0);
           if (PREFETCH && s == tid && pf_b == b) {
@@ -572,7 +597,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             py = pf_p[1];
             pz = pf_p[2];
           } else {
-            const unsigned g3 = 3u * (unsigned)at(gids, (unsigned)s);
+            const unsigned g3 = 3u * o;
             ux = at(A.x, g3);
             uy = at(A.x, g3 + 1);
             uz = at(A.x, g3 + 2);
@@ -582,13 +607,9 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
               pz = at(A.p, g3 + 2);
             }
           }
-          Vec4<X> u4 = {{ux, uy, uz, X(0)}};
-          *reinterpret_cast<Vec4<X>*>(u_lds + 4 * s) = u4;
-          if constexpr (NEEDV) {
-            Vec4<R> v4 = {{px, py, pz, R(0)}};
-            *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4;
-          }
-        }
+          put_u(s, Vec4<X>{{ux, uy, uz, X(0)}});
+          if constexpr (NEEDV) put_v(s, Vec4<R>{{px, py, pz, R(0)}});
+        });
       }
       __syncthreads();
 
