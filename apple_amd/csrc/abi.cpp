@@ -446,19 +446,19 @@ int elem_eval_impl(apl_mesh* m, int material, const void* mu, const void* lam, c
       const unsigned pw = passes[i];
       if (launch_elem(m, material, pw, mu, lam, u, nullptr, grad, hess_diag, acc, s, nullptr, ws))
         return -1;
-      if (launch_finish(m, pw, grad, hess_diag, (pw & W_E) ? energy : nullptr, nullptr, acc, nullptr, s, ws))
+      if (launch_finish(m, pw, grad, hess_diag, (pw & W_E) ? energy : nullptr, nullptr, acc, s, ws))
         return -1;
     }
   }
   if (w & W_HP) {
     if (launch_elem(m, material, W_HP, mu, lam, u, p, hess_prod, nullptr, acc, s, nullptr, ws))
       return -1;
-    if (launch_finish(m, W_HP, hess_prod, nullptr, nullptr, nullptr, acc, nullptr, s, ws)) return -1;
+    if (launch_finish(m, W_HP, hess_prod, nullptr, nullptr, nullptr, acc, s, ws)) return -1;
   }
   if (w & W_HQ) {
     if (launch_elem(m, material, W_HQ, mu, lam, u, p, nullptr, nullptr, acc, s, nullptr, ws))
       return -1;
-    if (launch_finish(m, W_HQ, nullptr, nullptr, nullptr, hess_quad, acc, nullptr, s, ws)) return -1;
+    if (launch_finish(m, W_HQ, nullptr, nullptr, nullptr, hess_quad, acc, s, ws)) return -1;
   }
   if (w & W_MIX) {
     if (launch_elem(m, material, W_MIX, mu, lam, u, p, dmu, dlam, acc, s, nullptr, ws))
@@ -584,8 +584,7 @@ int apl_bench_elem_pass(apl_mesh* m, int material, unsigned what, const void* mu
     for (int it = 0; it < iters && rc == 0; ++it) {
       rc = launch_elem(m, material, w, mu, lam, u, p, out_a, out_b, 0, s);
       if (rc == 0)
-        rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0,
-                           nullptr, s);
+        rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0, s);
     }
     APL_CHECK_HIP(hipEventRecord(ev[3], s));
   }
@@ -635,8 +634,7 @@ int apl_bench_elem_graph(apl_mesh* m, int material, unsigned what, const void* m
     for (int it = 0; it < iters && rc == 0; ++it) {
       rc = launch_elem(m, material, w, mu, lam, u, p, out_a, out_b, 0, cs);
       if (rc == 0)
-        rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0,
-                           nullptr, cs);
+        rc = launch_finish(m, w, out_a, out_b, (w & W_E) ? energy : nullptr, (w & W_HQ) ? energy : nullptr, 0, cs);
     }
     const hipError_t ec = hipStreamEndCapture(cs, &g);
     if (rc == 0 && ec == hipSuccess && g != nullptr &&

@@ -19,10 +19,8 @@ namespace apl {
 template <class R>
 struct FinishArgs {
   const int32_t* vblk_off;
-  const int32_t* vblk_inst;
   const int32_t* vtx_slot_off;
   const R* partial;
-  const int32_t* active;
   R* out_a;
   R* out_b;
   const double* blk_red;
@@ -32,14 +30,20 @@ struct FinishArgs {
   int ninst;  // instance workgroups (0: no energies / quadratic forms)
   int h_only;
   int accumulate;
+  int n_verts;
 };
 
-template <class R, int NCH>
+// The vertex sums wait for one chain, offsets -> partials -> sums.  FP32
+// passes of six channels on meshes of up to two vertex blocks per CU have all
+// of a thread's loads of the partials in flight at once (WINDOW: 45^3 5.3 ->
+// 4.3 us); with more blocks resident (64^3), three channels or FP64 the loop
+// of four is 0.2-0.4 us faster.  With one instance (SINGLE) the block's
+// vertices follow from its number.
+template <class R, int NCH, bool SINGLE, bool WINDOW>
 __global__ __launch_bounds__(NTH) void finish_kernel(FinishArgs<R> A) {
   __shared__ double eq[2 * (NTH / 64 + 1)];
   if ((int)blockIdx.x < A.ninst) {
     const int i = (int)blockIdx.x;
-    if (A.active != nullptr && A.active[i] == 0) return;
     const long long b0 = A.inst_blk_off[i];
     flat_column_sums<2, NTH>(A.blk_red + RED_STRIDE * b0, RED_STRIDE * (A.inst_blk_off[i + 1] - b0), eq);
     if (threadIdx.x == 0) {
@@ -50,10 +54,13 @@ __global__ __launch_bounds__(NTH) void finish_kernel(FinishArgs<R> A) {
   }
   if constexpr (NCH > 0) {
     const int vb = (int)blockIdx.x - A.ninst;
-    if (A.active != nullptr && A.active[A.vblk_inst[vb]] == 0) return;
     __shared__ R win[VSUM_LDS_BYTES / sizeof(R)];
-    const int v0 = A.vblk_off[vb], v1 = A.vblk_off[vb + 1];
+    const int v0 = SINGLE ? vb * NTH : A.vblk_off[vb];
+    const int v1 = SINGLE ? min(v0 + NTH, A.n_verts) : A.vblk_off[vb + 1];
     const int i0 = 3 * v0, i1 = 3 * v1;
+    VertexSums<R, NCH, NTH> vs{A.vtx_slot_off, A.partial, win};
+    typename VertexSums<R, NCH, NTH>::template Window<16> w;
+    if constexpr (WINDOW) vs.fetch(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R), w);
     int k0[DOF_PER_THREAD], k1[DOF_PER_THREAD];
 #pragma unroll
     for (int j = 0; j < DOF_PER_THREAD; ++j) {
@@ -64,8 +71,10 @@ __global__ __launch_bounds__(NTH) void finish_kernel(FinishArgs<R> A) {
         k1[j] = at(A.vtx_slot_off, (unsigned)(i / 3) + 1);
       }
     }
-    VertexSums<R, NCH, NTH> vs{A.vtx_slot_off, A.partial, win};
-    vs.stage(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R));
+    if constexpr (WINDOW)
+      vs.store(w);
+    else
+      vs.stage(v0, v1, VSUM_LDS_BYTES / (int)sizeof(R));
 #pragma unroll
     for (int j = 0; j < DOF_PER_THREAD; ++j) {
       const int i = i0 + (int)threadIdx.x + j * NTH;
@@ -199,7 +208,7 @@ int nloc_limit(int dtype) {
 }
 
 int launch_finish(apl_mesh* m, unsigned what, void* out_a, void* out_b, double* out_e, double* out_q,
-                  int accumulate, const int32_t* active, hipStream_t s, const Workspace* ws) {
+                  int accumulate, hipStream_t s, const Workspace* ws) {
   const bool g = what & W_G, h = what & W_H, hp = what & W_HP;
   const int nch = (g ? 3 : 0) + (h ? 3 : 0) + (hp ? 3 : 0);
   const bool inst = out_e != nullptr || out_q != nullptr;
@@ -211,10 +220,8 @@ int launch_finish(apl_mesh* m, unsigned what, void* out_a, void* out_b, double* 
     using R = std::remove_pointer_t<decltype(tag)>;
     FinishArgs<R> A;
     A.vblk_off = m->d.vblk_off;
-    A.vblk_inst = m->d.vblk_inst;
     A.vtx_slot_off = m->d.vtx_slot_off;
     A.partial = (const R*)(ws != nullptr ? ws->partial : m->d.partial);
-    A.active = active;
     A.out_a = (R*)out_a;
     A.out_b = (R*)out_b;
     A.blk_red = ws != nullptr ? ws->blk_red : m->d.blk_red;
@@ -224,7 +231,15 @@ int launch_finish(apl_mesh* m, unsigned what, void* out_a, void* out_b, double* 
     A.ninst = ninst;
     A.h_only = (h && !g && !hp) ? 1 : 0;
     A.accumulate = accumulate;
-    hipLaunchKernelGGL((finish_kernel<R, decltype(nch_c)::value>), dim3((unsigned)grid), dim3(NTH), 0, s, A);
+    A.n_verts = (int)m->L.V;
+    constexpr int NCH = decltype(nch_c)::value;
+    constexpr bool CAN_WINDOW = NCH == 6 && sizeof(R) == 4;
+    if (m->L.n_inst == 1 && CAN_WINDOW && nvblk <= 2 * m->n_cu)
+      hipLaunchKernelGGL((finish_kernel<R, NCH, true, CAN_WINDOW>), dim3((unsigned)grid), dim3(NTH), 0, s, A);
+    else if (m->L.n_inst == 1)
+      hipLaunchKernelGGL((finish_kernel<R, NCH, true, false>), dim3((unsigned)grid), dim3(NTH), 0, s, A);
+    else
+      hipLaunchKernelGGL((finish_kernel<R, NCH, false, false>), dim3((unsigned)grid), dim3(NTH), 0, s, A);
   };
   using I0 = std::integral_constant<int, 0>;
   using I3 = std::integral_constant<int, 3>;

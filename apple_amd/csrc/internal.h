@@ -122,7 +122,7 @@ int launch_elem(apl_mesh* m, int material, unsigned what, const void* mu, const 
 // when out_e / out_q are given, per-instance sums of the block energies /
 // quadratic forms.
 int launch_finish(apl_mesh* m, unsigned what, void* out_a, void* out_b, double* out_e, double* out_q,
-                  int accumulate, const int32_t* active, hipStream_t s, const Workspace* ws = nullptr);
+                  int accumulate, hipStream_t s, const Workspace* ws = nullptr);
 // material id valid for this mesh (APL_MODEL exactly for model meshes)
 bool material_ok(const apl_mesh* m, int material);
 // whether launches of this material read lambda

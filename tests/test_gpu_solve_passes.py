@@ -114,3 +114,23 @@ def test_a_mesh_without_tets_ends_at_once():
     st = DeviceSolver(pot).solve(x, None, None, PncgConfig())[0]
     assert st.success and st.n_steps == 0
     assert torch.equal(x, torch.full_like(x, 0.5))
+
+
+# the evaluation's vertex sums: one block, the largest and the next size whose partials are all in flight at
+# once (two vertex blocks per CU: 512), against the loop that a batch takes: the same sums, bit for bit
+@pytest.mark.parametrize("n", [2, 49, 50])
+def test_single_evaluation_equals_the_same_instance_of_a_batch(n):
+    print(f"[passes] evaluation n = {n}", flush=True)
+    m, fixed, x0, f = _case(n)
+    m2, fixed2, x2, f2 = _case(3, seed=1)
+    r, r2 = Region.from_mesh(m), Region.from_mesh(m2)
+    t = lambda a: torch.as_tensor(a, dtype=torch.float32, device="cuda").contiguous()  # noqa: E731
+    b = batch.Batch([batch.Instance(r2, m2.cell_data["mu"], m2.cell_data["lambda"], f2, fixed2, x2),
+                     batch.Instance(r, m.cell_data["mu"], m.cell_data["lambda"], f, fixed, x0)], _lib.APL_SNH, device="cuda")
+    pot = fem.StableNeoHookean.from_region(r, device="cuda")
+    g, h = torch.empty_like(t(x0)), torch.empty_like(t(x0))
+    pot.fused(t(x0), None, g, h, accumulate=False)
+    gb, hb = torch.empty_like(b.x0), torch.empty_like(b.x0)
+    b.mesh.eval(_lib.APL_SNH, b.mu, b.lam, torch.cat([t(x2), t(x0)]), grad=gb, hess_diag=hb)
+    assert torch.equal(b.split(gb)[1], g) and torch.equal(b.split(hb)[1], h)
+    assert g.abs().max() > 0 and h.abs().max() > 0
