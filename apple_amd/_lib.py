@@ -188,6 +188,34 @@ def lib():
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The extension module that calls the library from torch tensors
+    (csrc/python/tensor_calls.cpp) and the entries it calls, loaded once
+    (raises if it has not been built): (module, apl_elem_eval,
+    apl_elem_mixed_activation, apl_mesh_set_activation)."""
+    global _calls
+    if _calls is None:
+        import importlib.util
+
+        import torch  # noqa: F401  (the module is linked against its libraries)
+
+        L = lib()
+        path = os.path.join(os.path.dirname(LIB_PATH), "tensor_calls.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -m apple_amd.build`")
+        with _lock:
+            if _calls is None:
+                spec = importlib.util.spec_from_file_location("tensor_calls", path)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                _calls = (module, *(ctypes.cast(f, c_vp).value for f in (
+                    L.apl_elem_eval, L.apl_elem_mixed_activation, L.apl_mesh_set_activation)))
+    return _calls
+
+
 def check(rc: int) -> None:
     if rc != 0:
         raise RuntimeError("apple_amd: " + lib().apl_last_error().decode())

@@ -3,7 +3,8 @@
 Each ``csrc/*.hip`` and ``csrc/*.cpp`` file is compiled with hipcc in
 parallel and linked into one shared object with a C ABI (declared in
 ``include/apple_amd.h``).  Packed-FP32 instructions are disabled for all
-device code.
+device code.  ``csrc/python/tensor_calls.cpp`` becomes the extension module
+``apple_amd/_lib/tensor_calls.so`` (host code against PyTorch's headers).
 """
 
 from __future__ import annotations
@@ -13,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "_lib")
 OBJDIR = os.path.join(HERE, "_lib", "obj")
 LIBNAME = "libapple_amd.so"
+MODULE = "tensor_calls"
 ARCH = os.environ.get("APPLE_AMD_ARCH", "gfx950")
 
 DEVICE_FLAGS = [
@@ -52,13 +55,34 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_module() -> None:
+    """The extension module that calls the library from torch tensors."""
+    import torch
+    from torch.utils import cpp_extension
+
+    out = os.path.join(LIBDIR, MODULE + ".so")
+    include = [sysconfig.get_paths()["include"], *cpp_extension.include_paths()]
+    cmd = [
+        hipcc(), *COMMON, "-shared", os.path.join(CSRC, "python", MODULE + ".cpp"), "-o", out + ".tmp",
+        *(f"-isystem{p}" for p in include), f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+        *(f"-L{p}" for p in cpp_extension.library_paths()), "-lc10", "-ltorch_cpu", "-ltorch_python",
+    ]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+    os.replace(out + ".tmp", out)
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every source and link the shared library; returns its path."""
+    """Compile every source and link the shared library and the extension
+    module; returns the library's path."""
     os.makedirs(OBJDIR, exist_ok=True)
     srcs = sources()
-    jobs = min(len(srcs), max(1, min(16, os.cpu_count() or 1)))
+    jobs = min(len(srcs) + 1, max(1, min(16, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(jobs) as ex:
+        module = ex.submit(_build_module)
         objs = list(ex.map(_compile, srcs))
+        module.result()
     out = os.path.join(LIBDIR, LIBNAME)
     tmp = out + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]

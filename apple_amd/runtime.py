@@ -57,6 +57,11 @@ def current_stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+# The same for a device whose index is known and that is in use already
+# (no Stream object: 0.1 us instead of 1.9)
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 class DeviceMesh:
     """Owner of an ``apl_mesh`` handle: element data and the block partition.
 
@@ -143,6 +148,8 @@ class DeviceMesh:
                     _DT[self.dtype], T, self.n_verts, cells.ctypes.data, dminv.ctypes.data, dV.ctypes.data, *common,
                 )
             )
+        # what tensor_calls checks the tensors of a call against
+        self._spec = (int(self.dtype == torch.float64), self.device.index, self.n_tets, self.n_verts, self.n_inst)
         self._scratch = torch.zeros(max(self.n_inst, 1) * 2, dtype=torch.float64, device=self.device)
 
     @property
@@ -157,6 +164,12 @@ class DeviceMesh:
     def set_activation(self, activation: torch.Tensor | None) -> None:
         """Bind the (T, 6) activation that muscle-law launches read (the mesh
         keeps the pointer; this object keeps the tensor alive)."""
+        mod, _, _, entry = _lib.calls()
+        rc = mod.set_activation(entry, self._handle.value, 0, self._spec, activation)
+        if rc is not None:
+            _lib.check(rc)
+            self._activation = activation
+            return
         if activation is not None:
             ptr(activation, dtype=self.dtype, device=self.device, shape=(self.n_tets, 6), name="activation")
         _lib.check(_lib.lib().apl_mesh_set_activation(self._handle, activation.data_ptr() if activation is not None else None))
@@ -240,6 +253,14 @@ class DeviceMesh:
         accumulate=False,
     ) -> None:
         """One fused element pass writing (or adding into) the given outputs."""
+        mod, entry, _, _ = _lib.calls()
+        rc = mod.elem_eval(entry, self._handle.value, _raw_stream(self.device.index), self._spec, material, accumulate,
+                           mu, lam if material != _lib.APL_ARAP else None, u, p, energy, grad, hess_diag, hess_prod,
+                           hess_quad, dmu, dlam)
+        if rc is not None:
+            _lib.check(rc)
+            return
+        # an argument is not a plain tensor of the form it has to have: say which, or take it as it is
         what = 0
         if energy is not None:
             what |= _lib.APL_ENERGY
@@ -280,6 +301,12 @@ class DeviceMesh:
     def mixed_activation(self, mu, lam, u, p, dact, *, dmu=None, dlam=None, accumulate=False) -> None:
         """Muscle law: per-tet p^T d(grad)/d(activation) into dact (T, 6), and
         optionally p^T d(grad)/d(mu), d/d(lambda) in the same pass."""
+        mod, _, entry, _ = _lib.calls()
+        rc = mod.elem_mixed_activation(entry, self._handle.value, _raw_stream(self.device.index), self._spec,
+                                       accumulate, mu, lam, u, p, dact, dmu, dlam)
+        if rc is not None:
+            _lib.check(rc)
+            return
         tet = dict(dtype=self.dtype, device=self.device, shape=(self.n_tets,))
         _lib.check(
             _lib.lib().apl_elem_mixed_activation(
