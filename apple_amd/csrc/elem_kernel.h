@@ -99,10 +99,15 @@ struct alignas(2 * sizeof(T)) Vec2 {
 //            with W_VQ its d.Hd, so that the update needs no pass of its own
 //            for the step length
 //   W_ACT    the caller's direction, blocks of running instances only
+// W_ONE with W_TRIAL or W_DIR: the mesh has one instance, whose scalars each
+// workgroup reads once, by scalar loads (64^3: trial pass 31.0 -> 30.3 us,
+// direction pass 24.2 -> 23.7, against one variant for both; a batch's
+// direction pass grows from 24.6 to 26.6 us if it reads its states that way).
 // W_FUSED with one of them: a single instance's pass that takes the scalar
 // step before it (scalar_step).  A variant of its own: the batches' passes
 // lose 8-15 % to the registers and scalar traffic of that code.
-constexpr unsigned W_TRIAL = 256u, W_DIR = 512u, W_CGD = 1024u, W_ACT = 2048u, W_FUSED = 4096u;
+constexpr unsigned W_TRIAL = 256u, W_DIR = 512u, W_CGD = 1024u, W_ACT = 2048u, W_FUSED = 4096u,
+                   W_ONE = 8192u;
 constexpr unsigned W_SOLVER = W_TRIAL | W_DIR | W_CGD | W_ACT;
 constexpr unsigned W_OUT = 255u;  // the bits tet_eval knows
 constexpr unsigned OWNER_BIT = 0x80000000u;
@@ -142,6 +147,14 @@ __device__ __forceinline__ double uni(double v) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
+// Entry i of a table that the kernel does not write, i uniform: a scalar load
+// whatever the compiler knows of the kernel's stores.
+#define APL_CONSTANT __attribute__((address_space(4)))
+template <class T>
+__device__ __forceinline__ const APL_CONSTANT T& constant_at(const T* t, int i) {
+  return ((const APL_CONSTANT T*)(uintptr_t)t)[i];
+}
+
 struct InstScalars {
   double alpha, alpha_commit, beta, pmean;
   int act_eval, commit, act_dir, cur;
@@ -149,6 +162,9 @@ struct InstScalars {
   __device__ explicit InstScalars(const InstState& s)
       : alpha(uni(s.alpha)), alpha_commit(uni(s.alpha_commit)), beta(uni(s.beta)), pmean(uni(s.pmean)),
         act_eval(uni(s.act_eval)), commit(uni(s.commit)), act_dir(uni(s.act_dir)), cur(uni(s.cur)) {}
+  __device__ explicit InstScalars(const APL_CONSTANT InstState& s)
+      : alpha(s.alpha), alpha_commit(s.alpha_commit), beta(s.beta), pmean(s.pmean), act_eval(s.act_eval),
+        commit(s.commit), act_dir(s.act_dir), cur(s.cur) {}
 };
 
 // An accepted step: x += alpha_commit p, p = -P g + beta p with the Jacobi
@@ -166,11 +182,11 @@ struct Step {
   Vec4<double>* x1;
   Vec4<R>* p1;
   template <class State>
-  __device__ Step(const SolveArgs<R>& S, const State& st)
+  __device__ Step(const SolveArgs<R>& S, const State& st, int cur)
       : a(st.alpha_commit), beta((R)st.beta), ipm(R(1) / (R)st.pmean), dir(st.act_dir != 0),
-        x0(S.x + (st.cur ? (size_t)0 : S.V)), p0(S.p + (st.cur ? (size_t)0 : S.V)),
-        g(S.g + (st.cur ? S.V : (size_t)0)), P(S.P), x1(S.x + (st.cur ? S.V : (size_t)0)),
-        p1(S.p + (st.cur ? S.V : (size_t)0)) {}
+        x0(S.x + (cur ? (size_t)0 : S.V)), p0(S.p + (cur ? (size_t)0 : S.V)),
+        g(S.g + (cur ? S.V : (size_t)0)), P(S.P), x1(S.x + (cur ? S.V : (size_t)0)),
+        p1(S.p + (cur ? S.V : (size_t)0)) {}
 };
 
 // Element i of a uniform base pointer through a 32-bit byte offset: maps to
@@ -183,6 +199,68 @@ __device__ __forceinline__ const T& at(const T* base, unsigned i) {
 template <class T>
 __device__ __forceinline__ T& at(T* base, unsigned i) {
   return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + i * (unsigned)sizeof(T));
+}
+
+// 3 i: one full-rate instruction (a product with 12 or 24 compiles to a
+// 32-bit multiply, which takes four times as long).
+__device__ __forceinline__ unsigned three_times(unsigned i) {
+  unsigned t;
+  asm("v_lshl_add_u32 %0, %1, 1, %1" : "=v"(t) : "v"(i));
+  return t;
+}
+// Elements [N i, N i + N) of a uniform base pointer, N = 3 or 6, moved by the
+// widest accesses (dword alignment is enough for them).
+template <class T, int N>
+struct Run {
+  T v[N];
+};
+template <int N, class T>
+__device__ __forceinline__ const Run<T, N>& run_at(const T* base, unsigned i) {
+  static_assert(N == 3 || N == 6, "runs of three or six");
+  return *reinterpret_cast<const Run<T, N>*>(reinterpret_cast<const char*>(base) +
+                                            three_times(i) * (unsigned)(N / 3 * sizeof(T)));
+}
+template <int N, class T>
+__device__ __forceinline__ Run<T, N>& run_at(T* base, unsigned i) {
+  return const_cast<Run<T, N>&>(run_at<N>((const T*)base, i));
+}
+
+// LDS by byte address: base + SIZE * (the low or high half of w) in one
+// instruction each (as shifts, masks and adds two to three).
+#define APL_LDS __attribute__((address_space(3)))
+template <class T, int N>
+using Vx = T __attribute__((ext_vector_type(N)));
+__device__ __forceinline__ unsigned lds_address(const void* p) {
+  return (unsigned)(uintptr_t)(APL_LDS const char*)p;
+}
+template <class V>
+__device__ __forceinline__ V lds_get(unsigned a) {
+  return *(APL_LDS const V*)(uintptr_t)a;
+}
+// the first three of a padded vector
+template <class T>
+__device__ __forceinline__ V3<T> lds_get3(unsigned a) {
+  if constexpr (sizeof(T) == 8) {
+    const Vx<T, 2> w = lds_get<Vx<T, 2>>(a);  // (as one vector all 32 bytes are read)
+    return v3(w[0], w[1], lds_get<T>(a + 16));
+  } else {
+    const Vx<T, 3> w = lds_get<Vx<T, 3>>(a);
+    return v3(w[0], w[1], w[2]);
+  }
+}
+template <class V>
+__device__ __forceinline__ void lds_put(unsigned a, V v) {
+  *(APL_LDS V*)(uintptr_t)a = v;
+}
+template <int SIZE, bool HIGH>
+__device__ __forceinline__ unsigned lds_entry(unsigned w, unsigned base) {
+  static_assert(SIZE >= 4 && SIZE <= 64, "inline constants");
+  unsigned a;
+  if constexpr (HIGH)
+    asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(a) : "v"(w), "n"(SIZE), "s"(base));
+  else
+    asm("v_mad_u32_u16 %0, %1, %2, %3" : "=v"(a) : "v"(w), "n"(SIZE), "s"(base));
+  return a;
 }
 
 // Raw buffer loads: a scalar resource (base address) plus a per-lane and a
@@ -296,7 +374,7 @@ __device__ __forceinline__ void step_isolated(const SolveArgs<R>& S, const InstS
     if (s.commit == 0) continue;
     Vec4<double> u;
     Vec4<R> d;
-    step_vertex(Step<R>(S, s), (unsigned)S.iso[k], true, u, d);
+    step_vertex(Step<R>(S, s, s.cur), (unsigned)S.iso[k], true, u, d);
   }
 }
 
@@ -309,8 +387,8 @@ struct Direction {
   const Vec4<R>* d0;
   Vec4<R>* d1;
   template <class State>
-  __device__ Direction(const SolveArgs<R>& S, const State& st)
-      : beta((R)st.beta), z(S.z), d0(S.p + (st.cur ? (size_t)0 : S.V)), d1(S.p + (st.cur ? S.V : (size_t)0)) {}
+  __device__ Direction(const SolveArgs<R>& S, const State& st, int cur)
+      : beta((R)st.beta), z(S.z), d0(S.p + (cur ? (size_t)0 : S.V)), d1(S.p + (cur ? S.V : (size_t)0)) {}
 };
 
 template <class R>
@@ -328,7 +406,7 @@ __device__ __forceinline__ void direction_isolated(const SolveArgs<R>& S, const 
     const InstState& s = st[S.iso_inst[k]];
     if (s.act_eval == 0) continue;
     Vec4<R> d;
-    direction_vertex(Direction<R>(S, s), (unsigned)S.iso[k], true, d);
+    direction_vertex(Direction<R>(S, s, s.cur), (unsigned)S.iso[k], true, d);
   }
 }
 
@@ -392,6 +470,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   constexpr bool CGD = (WHAT & W_CGD) != 0;
   constexpr bool SOLVER = (WHAT & W_SOLVER) != 0;
   constexpr bool FUSED = (WHAT & W_FUSED) != 0;
+  constexpr bool ONE = FUSED || (WHAT & W_ONE) != 0;  // the mesh has one instance
   static_assert(SOLVER == !std::is_same_v<SOLVE, NoSolve>, "solver passes take SolveArgs");
   constexpr bool HAS_G = (WHAT & W_G) != 0;
   constexpr bool HAS_H = (WHAT & W_H) != 0;
@@ -415,6 +494,13 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   R* contrib = v_lds + (NEEDV ? 4 * A.nloc_max : 0);  // [channel group][position][channel in group]
   using PK = Pack<NCHA>;
 
+  // the same by LDS address: window slots and the two regions of the buffer
+  // (groups of four channels, the remainder)
+  const unsigned u_at = lds_address(u_lds), v_at = lds_address(v_lds), c_at = lds_address(contrib);
+  constexpr int GB = 4 * sizeof(R), RB = PK::REMW * sizeof(R);  // bytes per position
+  static_assert(PK::G4 <= 1, "one group of four channels");
+  const unsigned r_at = c_at + PK::G4 * GB * CS;
+
   const int tid = threadIdx.x;
   const int pid = blockIdx.x;
   const int xcd = pid & 7, k0 = pid >> 3, K = gridDim.x >> 3;
@@ -433,7 +519,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   auto xcd_block = [&](int j) {
     const int k = ((j / C) * 8 + xcd) * C + j % C;
     if constexpr (LIST)
-      return A.blk_list[k];
+      return constant_at(A.blk_list, k);
     else
       return k;
   };
@@ -442,7 +528,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   // only those of still-active instances.
   const int n_cand = k0 < nb_x ? (nb_x - k0 + K - 1) / K : 0;
   bool filter = false;
-  InstScalars single;  // the instance's scalars (FUSED)
+  InstScalars single;  // the instance's scalars (ONE)
   // the vertex of slot s of the block whose slots start at sb (with OWNER_BIT
   // where the pass needs it)
   auto slot_vertex = [&](int sb, int s) -> uint32_t {
@@ -459,8 +545,8 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   if constexpr (FUSED) {
     if (n_cand > 0) {
       pre_b = xcd_block(k0);
-      const int t0 = A.blk_tet_off[pre_b], t1 = A.blk_tet_off[pre_b + 1];
-      const int sb = A.blk_loc_off[pre_b], sb1 = A.blk_loc_off[pre_b + 1];
+      const int t0 = constant_at(A.blk_tet_off, pre_b), t1 = constant_at(A.blk_tet_off, pre_b + 1);
+      const int sb = constant_at(A.blk_loc_off, pre_b), sb1 = constant_at(A.blk_loc_off, pre_b + 1);
       pre_o = slot_vertex(sb, min(tid, sb1 - sb - 1));
       load_rec<MAT>(block_res<MAT>(A, t0), (unsigned)min(tid, t1 - t0 - 1), pre_rec);
     }
@@ -472,8 +558,13 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   } else if constexpr (SOLVER) {
     if constexpr (DIR) step_isolated(S, S.st);
     if constexpr (CGD) direction_isolated(S, S.st);
-    filter = S.filter != 0;
-    if (!filter && (DIR ? S.st[0].commit : S.st[0].act_eval) == 0) return;
+    if constexpr (ONE) {
+      single = InstScalars(constant_at(S.st, 0));
+      if ((DIR ? single.commit : single.act_eval) == 0) return;
+    } else {
+      filter = S.filter != 0;
+      if (!filter && (DIR ? S.st[0].commit : S.st[0].act_eval) == 0) return;
+    }
   }
   // the active-block list (solves only) sits after the contribution buffer
   int* act_list = reinterpret_cast<int*>(contrib + (SCATTER ? PK::NCHP * CS : 0));
@@ -490,15 +581,15 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       n_cand, filter, act_list, [&](int j) { return xcd_block(k0 + j * K); },
       [&](int bb) {
         if constexpr (SOLVER) {
-          const InstState& st = S.st[A.blk_inst[bb]];
+          const InstState& st = S.st[A.blk_inst[bb]];  // (bb differs by lane)
           return (DIR ? st.commit : st.act_eval) != 0;
         }
         return true;
       },
       [&](const int b, const int bn) {
       // the scalars of the block's instance
-      const auto& st = [&]() -> const auto& {
-        if constexpr (FUSED)
+      const auto& inst = [&]() -> const auto& {
+        if constexpr (ONE)
           return single;
         else if constexpr (SOLVER)
           return S.st[A.blk_inst[b]];
@@ -512,12 +603,20 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       // staging waits for the slot vertex alone.  With the destinations first
       // and each load under its own branch a block took five memory latencies
       // in turn, now three: 51^3 H v 27.6 -> 25.9 us, FP64 pass at 37^3 25.9 ->
-      // 24.4 us, 64^3 solve 55.6 -> 53.1 ms.
-      const int t0 = A.blk_tet_off[b], t1 = A.blk_tet_off[b + 1];
-      const int sb = A.blk_loc_off[b], sb1 = A.blk_loc_off[b + 1];
+      // 24.4 us, 64^3 solve 55.6 -> 53.1 ms.  The positions of the slots come
+      // along (looked up after the staging they were a latency of their own);
+      // with that, fewer address instructions and one barrier less per block
+      // 51^3 H v 25.8 -> 22.6 us, 45^3 muscle 22.0 -> 20.1, 64^3 SNH 40.7 -> 39.1,
+      // ARAP 52.3 -> 50.5 (whole evaluations).
+      const int t0 = constant_at(A.blk_tet_off, b), t1 = constant_at(A.blk_tet_off, b + 1);
+      const int sb = constant_at(A.blk_loc_off, b), sb1 = constant_at(A.blk_loc_off, b + 1);
+      const int co_off = SCATTER ? constant_at(A.blk_co_off, b) : 0;
       const int nt = t1 - t0, nloc = sb1 - sb;
       const int lg = (4 * nloc <= SPT * NTH) ? 2 : ((2 * nloc <= SPT * NTH) ? 1 : 0);
       const int tps = 1 << lg;
+      // which of its two buffers the instance is in: the staging's addresses wait for it
+      int cur = 0;
+      if constexpr (TRIAL || DIR || CGD) cur = inst.cur;
       const BlockRes br = block_res<MAT>(A, t0);
       uint32_t o0 = pre_o;
       TetRec<R> rec;
@@ -529,14 +628,23 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         load_rec<MAT>(br, (unsigned)min(tid, nt - 1), rec);
       }
       int dst_pre[SPT];
+      uint32_t run_pre[SPT];  // the first chunk's positions of the slot item: [low half, high half)
+      const uint16_t* co = A.chunk_off + co_off;
+      auto slot_run = [&](const uint16_t* cc, int s) {
+        uint32_t w;
+        __builtin_memcpy(&w, &at(cc, (unsigned)s), sizeof(w));  // entries s and s + 1
+        return w;
+      };
       if constexpr (SCATTER) {
 #pragma unroll
-        for (int k = 0; k < SPT; ++k)
-          dst_pre[k] = at(A.loc_dst + sb, (unsigned)min((tid + k * NTH) >> lg, nloc - 1));
+        for (int k = 0; k < SPT; ++k) {
+          const int s = min((tid + k * NTH) >> lg, nloc - 1);
+          dst_pre[k] = at(A.loc_dst + sb, (unsigned)s);
+          run_pre[k] = slot_run(co, s);
+        }
       }
-      // (a vertex is never all ones; asked here, or the compiler moves the load of
-      // o0 down into the staging's branch, behind the others)
-      const int s_first = o0 != ~0u ? tid : nloc;
+      // (a lane's own value from here: made uniform where it is loaded, it is waited for there)
+      if constexpr (SOLVER && !ONE) asm("" : "+v"(cur));
 
       // stage the block's vertex window (u = x + alpha p for a trial point; the
       // new iterate and direction for an accepted step): stage(slot, o), o its
@@ -545,16 +653,16 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       auto put_v = [&](int s, const Vec4<R>& v4) { *reinterpret_cast<Vec4<R>*>(v_lds + 4 * s) = v4; };
       auto window = [&](auto stage) {
         // the thread's first slot apart from the others, or the wait at the
-        // loop's head would be for the tet records too; and a vertex is never
-        // all ones: asked here, so that the load of o0 is not moved down into
-        // this branch, behind the others
-        if (tid < nloc && o0 != ~0u) {
+        // loop's head would be for the tet records too; and neither a vertex
+        // nor cur is ever all ones: asked here, so that their loads are not
+        // moved down into this branch, behind the others
+        if ((tid < nloc) & (o0 != ~0u) & (cur != -1)) {
           stage(tid, o0);
           for (int s = tid + NTH; s < nloc; s += NTH) stage(s, slot_vertex(sb, s));
         }
       };
       if constexpr (DIR) {
-        const Step<R> step(S, st);
+        const Step<R> step(S, inst, cur);
         window([&](int s, uint32_t o) {
           Vec4<X> u4;
           Vec4<R> v4;
@@ -564,19 +672,20 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
         });
         if (!step.dir) return;  // converged at this step: no new direction
       } else if constexpr (CGD) {
-        const Direction<R> dir(S, st);
+        const Direction<R> dir(S, inst, cur);
         window([&](int s, uint32_t o) {
           const unsigned v = o & ~OWNER_BIT;
-          const Vec4<X> u4 = {{at(A.x, 3u * v), at(A.x, 3u * v + 1), at(A.x, 3u * v + 2), X(0)}};
+          const auto xv = run_at<3>(A.x, v);
+          const Vec4<X> u4 = {{xv.v[0], xv.v[1], xv.v[2], X(0)}};
           Vec4<R> v4;
           direction_vertex(dir, v, (o & OWNER_BIT) != 0, v4);
           put_u(s, u4);
           put_v(s, v4);
         });
       } else if constexpr (TRIAL) {
-        const double alpha = st.alpha;
-        const Vec4<double>* xb = S.x + (st.cur ? S.V : (size_t)0);
-        const Vec4<R>* pb = S.p + (st.cur ? S.V : (size_t)0);
+        const double alpha = inst.alpha;
+        const Vec4<double>* xb = S.x + (cur ? S.V : (size_t)0);
+        const Vec4<R>* pb = S.p + (cur ? S.V : (size_t)0);
         window([&](int s, uint32_t o) {
           const size_t v = o;
           Vec4<double> u4 = xb[v];
@@ -597,14 +706,15 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             py = pf_p[1];
             pz = pf_p[2];
           } else {
-            const unsigned g3 = 3u * o;
-            ux = at(A.x, g3);
-            uy = at(A.x, g3 + 1);
-            uz = at(A.x, g3 + 2);
+            const auto xv = run_at<3>(A.x, o);
+            ux = xv.v[0];
+            uy = xv.v[1];
+            uz = xv.v[2];
             if constexpr (NEEDV) {
-              px = at(A.p, g3);
-              py = at(A.p, g3 + 1);
-              pz = at(A.p, g3 + 2);
+              const auto pv = run_at<3>(A.p, o);
+              px = pv.v[0];
+              py = pv.v[1];
+              pz = pv.v[2];
             }
           }
           put_u(s, Vec4<X>{{ux, uy, uz, X(0)}});
@@ -619,44 +729,52 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
 #pragma unroll
         for (int ch = 0; ch < NCHA; ++ch) acc[k][ch] = R(0);
       R e_acc = R(0), q_acc = R(0);
-      const uint16_t* co = A.chunk_off + A.blk_co_off[b];
+      // one FP64 partial per wave and column into LDS, added in a fixed order
+      // by one thread after the next barrier
+      auto wave_partials = [&]() {
+        const int lane = tid & 63, w = tid >> 6;
+        if constexpr ((WHAT & W_E) != 0) {
+          const double e = wave_sum((double)e_acc);
+          if (lane == 63) red[2 * w] = e;
+        }
+        if constexpr (RED_Q) {
+          const double q = wave_sum((double)q_acc);
+          if (lane == 63) red[2 * w + 1] = q;
+        }
+      };
+      // before the sums of the slots, where its chain overlaps the LDS writes
+      // (64^3 SNH 39.75 -> 39.4 us), but not when the waves come to that
+      // barrier at different times (ARAP: 50.3 us after them, 51.2 before)
+      constexpr bool EARLY_RED = RED && MAT != MAT_ARAP;
       const int nchunks = (nt + NTH - 1) / NTH;
       for (int c = 0; c < nchunks; ++c) {
         const int tl = c * NTH + tid;
         // this chunk's position ranges of the thread's slot items
-        int q0[SPT], q1[SPT];
+        uint32_t runs[SPT];
         if constexpr (SCATTER) {
-          const uint16_t* cc = co + c * (nloc + 1);
 #pragma unroll
-          for (int k = 0; k < SPT; ++k) {
-            const int item = tid + k * NTH;
-            const int s = item >> lg;
-            q0[k] = 0;
-            q1[k] = 0;
-            if (s < nloc) {
-              q0[k] = at(cc, (unsigned)s) + (item & (tps - 1));
-              q1[k] = at(cc, (unsigned)s + 1);
-            }
-          }
+          for (int k = 0; k < SPT; ++k)
+            runs[k] = c == 0 ? run_pre[k] : slot_run(co + c * (nloc + 1), min((tid + k * NTH) >> lg, nloc - 1));
         }
         if (tl < nt) {
           if (c > 0) load_rec<MAT>(br, (unsigned)tl, rec);
           const TetGeom<R> g = make_geom(rec.B, rec.dV);
-          const int sidx[4] = {(int)(rec.cr.x & 0xffffu), (int)(rec.cr.x >> 16), (int)(rec.cr.y & 0xffffu),
-                               (int)(rec.cr.y >> 16)};
           // edge differences u_a - u_0 in the storage precision X, then R: F - I
           // depends only on them, and forming them before rounding keeps F
           // accurate relative to the strain rather than to |u|.
-          Vec4<X> uc[4];
+          constexpr int XB = 4 * sizeof(X), VB = 4 * sizeof(R);  // bytes per window slot
+          const unsigned ua[4] = {lds_entry<XB, false>(rec.cr.x, u_at), lds_entry<XB, true>(rec.cr.x, u_at),
+                                  lds_entry<XB, false>(rec.cr.y, u_at), lds_entry<XB, true>(rec.cr.y, u_at)};
+          V3<X> uc[4];
 #pragma unroll
-          for (int a = 0; a < 4; ++a) uc[a] = *reinterpret_cast<const Vec4<X>*>(u_lds + 4 * sidx[a]);
+          for (int a = 0; a < 4; ++a) uc[a] = lds_get3<X>(ua[a]);
           V3<R> u[4], v[4];
 #pragma unroll
           for (int a = 0; a < 4; ++a) {
-            u[a] = v3((R)(uc[a].v[0] - uc[0].v[0]), (R)(uc[a].v[1] - uc[0].v[1]), (R)(uc[a].v[2] - uc[0].v[2]));
+            u[a] = v3((R)(uc[a].x - uc[0].x), (R)(uc[a].y - uc[0].y), (R)(uc[a].z - uc[0].z));
             if constexpr (NEEDV) {
-              const Vec4<R> vv = *reinterpret_cast<const Vec4<R>*>(v_lds + 4 * sidx[a]);
-              v[a] = v3(vv.v[0], vv.v[1], vv.v[2]);
+              const uint32_t w = a < 2 ? rec.cr.x : rec.cr.y;
+              v[a] = lds_get3<R>(a % 2 ? lds_entry<VB, true>(w, v_at) : lds_entry<VB, false>(w, v_at));
             } else {
               v[a] = v3(R(0), R(0), R(0));
             }
@@ -688,8 +806,6 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             }
           }
           if constexpr (SCATTER) {
-            const int pos[4] = {(int)(rec.cr.z & 0xffffu), (int)(rec.cr.z >> 16), (int)(rec.cr.w & 0xffffu),
-                                (int)(rec.cr.w >> 16)};
 #pragma unroll
             for (int a = 0; a < 4; ++a) {
               R vals[NCHA];
@@ -711,85 +827,97 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
                 vals[ch + 1] = o.hp[a].y;
                 vals[ch + 2] = o.hp[a].z;
               }
-#pragma unroll
-              for (int gi = 0; gi < PK::G4; ++gi) {
-                const Vec4<R> t = {{vals[4 * gi], vals[4 * gi + 1], vals[4 * gi + 2], vals[4 * gi + 3]}};
-                *reinterpret_cast<Vec4<R>*>(contrib + gi * 4 * CS + 4 * pos[a]) = t;
-              }
-              R* rem = contrib + PK::G4 * 4 * CS;
+              const uint32_t w = a < 2 ? rec.cr.z : rec.cr.w;  // the corner's position
+              if constexpr (PK::G4 > 0)
+                lds_put(a % 2 ? lds_entry<GB, true>(w, c_at) : lds_entry<GB, false>(w, c_at),
+                        Vx<R, 4>{vals[0], vals[1], vals[2], vals[3]});
               constexpr int c0 = 4 * PK::G4;
-              if constexpr (PK::REM == 3) {
-                const Vec4<R> t = {{vals[c0], vals[c0 + 1], vals[c0 + 2], R(0)}};
-                *reinterpret_cast<Vec4<R>*>(rem + 4 * pos[a]) = t;
-              } else if constexpr (PK::REM == 2) {
-                const Vec2<R> t = {{vals[c0], vals[c0 + 1]}};
-                *reinterpret_cast<Vec2<R>*>(rem + 2 * pos[a]) = t;
-              } else if constexpr (PK::REM == 1) {
-                rem[pos[a]] = vals[c0];
+              if constexpr (PK::REM > 0) {
+                const unsigned ra = a % 2 ? lds_entry<RB, true>(w, r_at) : lds_entry<RB, false>(w, r_at);
+                if constexpr (PK::REM == 3)
+                  lds_put(ra, Vx<R, 4>{vals[c0], vals[c0 + 1], vals[c0 + 2], R(0)});
+                else if constexpr (PK::REM == 2)
+                  lds_put(ra, Vx<R, 2>{vals[c0], vals[c0 + 1]});
+                else
+                  lds_put(ra, vals[c0]);
               }
             }
           }
         }
+        if constexpr (EARLY_RED)
+          if (c == nchunks - 1) wave_partials();
+        if constexpr (SCATTER) __syncthreads();
         if constexpr (SCATTER) {
-          __syncthreads();
+          // one position's channels: a 4-channel group per 16/32-byte load, then the remainder
+          auto load_pos = [&](unsigned ga, unsigned ra, R (&t)[PK::NCHP]) {
+            if constexpr (PK::G4 > 0) {
+              const Vx<R, 4> w = lds_get<Vx<R, 4>>(ga);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) t[i] = w[i];
+            }
+            constexpr int c0 = 4 * PK::G4;
+            if constexpr (PK::REM == 3) {
+              const V3<R> w = lds_get3<R>(ra);
+              t[c0] = w.x;
+              t[c0 + 1] = w.y;
+              t[c0 + 2] = w.z;
+            } else if constexpr (PK::REM == 2) {
+              const Vx<R, 2> w = lds_get<Vx<R, 2>>(ra);
+              t[c0] = w[0];
+              t[c0 + 1] = w[1];
+            } else if constexpr (PK::REM == 1) {
+              t[c0] = lds_get<R>(ra);
+            }
+          };
 #pragma unroll
           for (int k = 0; k < SPT; ++k) {
-            // one position's channels: a 4-channel group per 16/32-byte load, then the remainder
-            auto load_pos = [&](int q, R (&t)[PK::NCHP]) {
-#pragma unroll
-              for (int gi = 0; gi < PK::G4; ++gi) {
-                const Vec4<R> w = *reinterpret_cast<const Vec4<R>*>(contrib + gi * 4 * CS + 4 * q);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) t[4 * gi + i] = w.v[i];
-              }
-              const R* rem = contrib + PK::G4 * 4 * CS;
-              constexpr int c0 = 4 * PK::G4;
-              if constexpr (PK::REM == 3) {
-                const Vec4<R> w = *reinterpret_cast<const Vec4<R>*>(rem + 4 * q);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) t[c0 + i] = w.v[i];
-              } else if constexpr (PK::REM == 2) {
-                const Vec2<R> w = *reinterpret_cast<const Vec2<R>*>(rem + 2 * q);
-                t[c0] = w.v[0];
-                t[c0 + 1] = w.v[1];
-              } else if constexpr (PK::REM == 1) {
-                t[c0] = rem[q];
-              }
-            };
-            int q = q0[k];
-            // two positions per step, both loads first; the sums keep the sequential order
-            for (; q + tps < q1[k]; q += 2 * tps) {
+            const int item = tid + k * NTH;
+            const bool mine = (item >> lg) < nloc;
+            const int q = mine ? (int)(runs[k] & 0xffffu) + (item & (tps - 1)) : 0;
+            const int q1 = mine ? (int)(runs[k] >> 16) : 0;
+            // two positions per step, both loads first, each with its own address
+            // (they advance by a uniform stride); the sums keep the sequential order
+            int n = q1 - q;
+            unsigned ga = c_at + (unsigned)GB * (unsigned)q, ra = r_at + (unsigned)RB * (unsigned)q;
+            unsigned gb = ga + (unsigned)GB * tps, rb = ra + (unsigned)RB * tps;
+            for (; n > tps; n -= 2 * tps) {
               R ta[PK::NCHP], tb[PK::NCHP];
-              load_pos(q, ta);
-              load_pos(q + tps, tb);
+              load_pos(ga, ra, ta);
+              load_pos(gb, rb, tb);
+              ga += 2 * GB * tps;
+              gb += 2 * GB * tps;
+              ra += 2 * RB * tps;
+              rb += 2 * RB * tps;
 #pragma unroll
               for (int ch = 0; ch < NCH; ++ch) acc[k][ch] = (acc[k][ch] + ta[ch]) + tb[ch];
             }
-            if (q < q1[k]) {
+            if (n > 0) {
               R ta[PK::NCHP];
-              load_pos(q, ta);
+              load_pos(ga, ra, ta);
 #pragma unroll
               for (int ch = 0; ch < NCH; ++ch) acc[k][ch] += ta[ch];
             }
           }
-          __syncthreads();
         }
+        if constexpr (RED && !EARLY_RED)
+          if (c == nchunks - 1) wave_partials();
+        if constexpr (SCATTER || RED) __syncthreads();
       }
 
       if constexpr (PREFETCH) {
         if (bn >= 0) {
-          const int sb_n = A.blk_loc_off[bn];
-          const int nloc_n = A.blk_loc_off[bn + 1] - sb_n;
+          const int sb_n = constant_at(A.blk_loc_off, bn);
+          const int nloc_n = constant_at(A.blk_loc_off, bn + 1) - sb_n;
           pf_b = bn;
           if (tid < nloc_n) {
-            const unsigned g3 = 3u * (unsigned)at(A.loc_gid + sb_n, (unsigned)tid);
-            pf_x[0] = at(A.x, g3);
-            pf_x[1] = at(A.x, g3 + 1);
-            pf_x[2] = at(A.x, g3 + 2);
+            const unsigned v = (unsigned)at(A.loc_gid + sb_n, (unsigned)tid);
+            const auto xv = run_at<3>(A.x, v);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) pf_x[k] = xv.v[k];
             if constexpr (NEEDV) {
-              pf_p[0] = at(A.p, g3);
-              pf_p[1] = at(A.p, g3 + 1);
-              pf_p[2] = at(A.p, g3 + 2);
+              const auto pv = run_at<3>(A.p, v);
+#pragma unroll
+              for (int k = 0; k < 3; ++k) pf_p[k] = pv.v[k];
             }
           }
         }
@@ -814,27 +942,16 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           const int item = tid + k * NTH;
           const int s = item >> lg;
           if (s < nloc && (item & (tps - 1)) == 0) {
-            const unsigned j = (unsigned)dst_pre[k] * NCH;
+            // (by element: a store of the whole record could be one to the block
+            // tables for all the compiler knows, whose loads would no longer be scalar)
+            auto& sums = run_at<NCH>(A.partial, (unsigned)dst_pre[k]);
 #pragma unroll
-            for (int ch = 0; ch < NCH; ++ch) at(A.partial, j + ch) = acc[k][ch];
+            for (int ch = 0; ch < NCH; ++ch) sums.v[ch] = acc[k][ch];
           }
         }
       }
       if constexpr (RED) {
-        // one FP64 partial per wave and column into LDS; thread 0 adds them
-        // in a fixed order after one barrier (the block's closing barrier
-        // keeps red from being overwritten before it has read it)
-        const int lane = tid & 63, w = tid >> 6;
-        if constexpr ((WHAT & W_E) != 0) {
-          const double e = wave_sum((double)e_acc);
-          if (lane == 63) red[2 * w] = e;
-        }
-        if constexpr (RED_Q) {
-          const double q = wave_sum((double)q_acc);
-          if (lane == 63) red[2 * w + 1] = q;
-        }
-        __syncthreads();
-        if (tid == 0) {
+        if (tid == NTH - 64) {  // of the last wave, whose lanes have the fewest slots
 #pragma unroll
           for (int col = 0; col < 2; ++col) {
             if (col == 0 && (WHAT & W_E) == 0) continue;
@@ -849,7 +966,11 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           }
         }
       }
-      __syncthreads();
+      // The next block's window may overwrite this one's: its readers are past
+      // the barrier after the tets (the mixed passes have none).  The wave
+      // partials and the contributions are written again only after the next
+      // window's barrier.
+      if constexpr (!SCATTER && !RED) __syncthreads();
       });
 }
 
@@ -949,6 +1070,7 @@ constexpr auto pass_kernel() {
 constexpr int variant_index(unsigned what) {
   constexpr unsigned v[N_VARIANTS] = {W_E, W_E | W_G | W_H, W_G, W_H, W_HP, W_HQ, W_MIX, W_MIXA, W_MIX | W_MIXA,
                                       W_E | W_G | W_H | W_TRIAL, W_HQ | W_DIR, W_HP | W_VQ | W_CGD, W_HP | W_ACT,
+                                      W_E | W_G | W_H | W_TRIAL | W_ONE, W_HQ | W_DIR | W_ONE,
                                       W_E | W_G | W_H | W_TRIAL | W_FUSED, W_HQ | W_DIR | W_FUSED,
                                       W_HP | W_VQ | W_CGD | W_FUSED};
   for (int i = 0; i < N_VARIANTS; ++i)

@@ -16,7 +16,7 @@ constexpr int NTH = 256;       // threads per element / vector block
 constexpr int MAX_CH = 6;      // scatter channels per incidence (grad + hdiag)
 constexpr int N_DOTS = 16;     // per vertex-block partial dot products
 constexpr int RED_STRIDE = 2;  // per element block: energy, quadratic form
-constexpr int N_VARIANTS = 16;  // element pass variants (elem_kernel.h, variant_index)
+constexpr int N_VARIANTS = 18;  // element pass variants (elem_kernel.h, variant_index)
 // material id of a model mesh's launches: every law over its own blocks
 constexpr int MAT_MODEL = 3;
 

@@ -7,17 +7,18 @@
 namespace apl {
 
 // Moves by DPP.
-// Lanes whose DPP source does not exist (row_shr at a row start, rows the
-// row mask leaves out) read `old` = 0.
+// Lanes whose DPP source does not exist read 0: at a row's start by the bound
+// control, in rows that the row mask leaves out from `old` (which takes an
+// instruction to clear, so bound control wherever no row is left out).
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ float dpp_f32(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, false));
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xF, ROW_MASK == 0xF));
 }
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ double dpp_f64(double v) {
   const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, ROW_MASK, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xF, false);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, ROW_MASK, 0xF, ROW_MASK == 0xF);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROW_MASK, 0xF, ROW_MASK == 0xF);
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 template <class T, int CTRL, int ROW_MASK = 0xF>

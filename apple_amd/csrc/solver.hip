@@ -741,7 +741,8 @@ static int pncg_iteration(apl_solver* s, const void* mu, const void* lam, const 
   } else {
     hipLaunchKernelGGL(pncg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sb, sa, P, s->hq, m->d.inst_blk_off);
     S.st = sa;
-    rc = launch_solve_pass<PASS_TRIAL, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+    rc = ni == 1 ? launch_solve_pass<PASS_TRIAL | W_ONE, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st)
+                 : launch_solve_pass<PASS_TRIAL, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
   }
   if (rc) return -1;
   if (nvb && ni == 1)
@@ -756,7 +757,8 @@ static int pncg_iteration(apl_solver* s, const void* mu, const void* lam, const 
   } else {
     hipLaunchKernelGGL(pncg_scalar_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sa, sb, P, m->d.vblk_dots, m->d.inst_vblk_off);
     S.st = sb;
-    rc = launch_solve_pass<PASS_DIR, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
+    rc = ni == 1 ? launch_solve_pass<PASS_DIR | W_ONE, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st)
+                 : launch_solve_pass<PASS_DIR, R>(m, s->material, mu, lam, nullptr, nullptr, S, grid, st);
   }
   if (rc) return -1;
   APL_CHECK_HIP(hipGetLastError());
@@ -828,6 +830,8 @@ static int pncg_begin_t(apl_solver* s, const void* mu, const void* lam, void* x,
   // occupancy-derived grids are queried (and cached) outside any capture
   solve_pass_grid<PASS_TRIAL, R>(m, s->material);
   solve_pass_grid<PASS_DIR, R>(m, s->material);
+  solve_pass_grid<PASS_TRIAL | W_ONE, R>(m, s->material);
+  solve_pass_grid<PASS_DIR | W_ONE, R>(m, s->material);
   solve_pass_grid<PASS_TRIAL | W_FUSED, R>(m, s->material);
   solve_pass_grid<PASS_DIR | W_FUSED, R>(m, s->material);
   // cached graph of K iterations for these pointers and parameters
