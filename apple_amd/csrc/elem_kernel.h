@@ -705,6 +705,20 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             px = pf_p[0];
             py = pf_p[1];
             pz = pf_p[2];
+          } else if constexpr (PREFETCH) {
+            // (a load per component, as the prefetch: one for all three lands in
+            // registers of its own, and the prefetched values would be waited
+            // for where they are loaded, to be moved there: 64^3 v.Hv 22.1 ->
+            // 26.3 us)
+            const unsigned g3 = 3u * o;
+            ux = at(A.x, g3);
+            uy = at(A.x, g3 + 1);
+            uz = at(A.x, g3 + 2);
+            if constexpr (NEEDV) {
+              px = at(A.p, g3);
+              py = at(A.p, g3 + 1);
+              pz = at(A.p, g3 + 2);
+            }
           } else {
             const auto xv = run_at<3>(A.x, o);
             ux = xv.v[0];
@@ -745,7 +759,7 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       // before the sums of the slots, where its chain overlaps the LDS writes
       // (64^3 SNH 39.75 -> 39.4 us), but not when the waves come to that
       // barrier at different times (ARAP: 50.3 us after them, 51.2 before)
-      constexpr bool EARLY_RED = RED && MAT != MAT_ARAP;
+      constexpr bool EARLY_RED = RED && SCATTER && MAT != MAT_ARAP;
       const int nchunks = (nt + NTH - 1) / NTH;
       for (int c = 0; c < nchunks; ++c) {
         const int tl = c * NTH + tid;
@@ -899,9 +913,9 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             }
           }
         }
-        if constexpr (RED && !EARLY_RED)
+        if constexpr (RED && SCATTER && !EARLY_RED)
           if (c == nchunks - 1) wave_partials();
-        if constexpr (SCATTER || RED) __syncthreads();
+        if constexpr (SCATTER) __syncthreads();
       }
 
       if constexpr (PREFETCH) {
@@ -910,14 +924,14 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
           const int nloc_n = constant_at(A.blk_loc_off, bn + 1) - sb_n;
           pf_b = bn;
           if (tid < nloc_n) {
-            const unsigned v = (unsigned)at(A.loc_gid + sb_n, (unsigned)tid);
-            const auto xv = run_at<3>(A.x, v);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) pf_x[k] = xv.v[k];
+            const unsigned g3 = 3u * (unsigned)at(A.loc_gid + sb_n, (unsigned)tid);
+            pf_x[0] = at(A.x, g3);
+            pf_x[1] = at(A.x, g3 + 1);
+            pf_x[2] = at(A.x, g3 + 2);
             if constexpr (NEEDV) {
-              const auto pv = run_at<3>(A.p, v);
-#pragma unroll
-              for (int k = 0; k < 3; ++k) pf_p[k] = pv.v[k];
+              pf_p[0] = at(A.p, g3);
+              pf_p[1] = at(A.p, g3 + 1);
+              pf_p[2] = at(A.p, g3 + 2);
             }
           }
         }
@@ -949,6 +963,10 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
             for (int ch = 0; ch < NCH; ++ch) sums.v[ch] = acc[k][ch];
           }
         }
+      }
+      if constexpr (RED && !SCATTER) {  // behind the prefetch, whose latency this hides
+        wave_partials();
+        __syncthreads();
       }
       if constexpr (RED) {
         if (tid == NTH - 64) {  // of the last wave, whose lanes have the fewest slots
