@@ -314,20 +314,35 @@ __global__ __launch_bounds__(SCAL_TH) void pncg_scalar_kernel(const InstState* i
   out[i] = s;
 }
 
+// An instance's state on its way through a scalar kernel: into LDS (one double
+// per thread, stored before the sums, whose barriers publish it), and out again
+// after thread 0's step.  As a local of thread 0 that only the step touches it
+// was given to every thread, in scratch and 49 KB of LDS: the alpha kernel of
+// 256 instances took 17 us instead of 4.5.
+__device__ __forceinline__ void state_in(const InstState* in, InstState* lds) {
+  const int t = threadIdx.x;
+  if (t < STATE_DOUBLES) reinterpret_cast<double*>(lds)[t] = reinterpret_cast<const double*>(in)[t];
+}
+template <class Step>
+__device__ __forceinline__ void state_out(InstState* lds, InstState* out, Step step) {
+  const int t = threadIdx.x;
+  if (t == 0) step(*lds);
+  __syncthreads();
+  if (t < STATE_DOUBLES) reinterpret_cast<double*>(out)[t] = reinterpret_cast<const double*>(lds)[t];
+}
+
 // S2: alpha from the quadratic form; clears the per-iteration flags
 __global__ __launch_bounds__(SCAL_TH) void pncg_alpha_kernel(const InstState* in, InstState* out, Params P,
                                                          const double* hq, const int64_t* inst_blk_off) {
   __shared__ double red[SCAL_TH / 64];
   const int i = blockIdx.x;
   // all loads issued before the first wait, as in pncg_scalar_kernel
+  __shared__ InstState s;
   const bool dir = in[i].act_dir != 0;
   const long long b0 = inst_blk_off[i], b1 = inst_blk_off[i + 1];
-  InstState s;
-  if (threadIdx.x == 0) s = in[i];
+  state_in(in + i, &s);
   const double q = flat_sum_odd<SCAL_TH>(hq + b0, dir ? b1 - b0 : 0, red);
-  if (threadIdx.x != 0) return;
-  pncg_alpha_step(s, P, q);
-  out[i] = s;
+  state_out(&s, out + i, [&](InstState& st) { pncg_alpha_step(st, P, q); });
 }
 
 // ------------------------------------------------------------------ PCG (adjoint)
@@ -495,12 +510,10 @@ __global__ __launch_bounds__(SCAL_TH) void cg_beta_kernel(const InstState* in, I
   // all loads issued before the first wait, as in pncg_scalar_kernel
   const bool act = in[i].act_eval != 0;
   const long long vb0 = inst_vblk_off[i], vb1 = inst_vblk_off[i + 1];
-  InstState s;
-  if (threadIdx.x == 0) s = in[i];
+  __shared__ InstState s;
+  state_in(in + i, &s);
   flat_column_sums<2, SCAL_TH>(dots + 2 * vb0, act ? 2 * (vb1 - vb0) : 0, tot);
-  if (threadIdx.x != 0) return;
-  cg_beta_step(s, rtol, max_iters, tot[0], tot[1]);
-  out[i] = s;
+  state_out(&s, out + i, [&](InstState& st) { cg_beta_step(st, rtol, max_iters, tot[0], tot[1]); });
 }
 
 __global__ __launch_bounds__(SCAL_TH) void cg_alpha_kernel(const InstState* in, InstState* out, const double* table,
@@ -509,12 +522,10 @@ __global__ __launch_bounds__(SCAL_TH) void cg_alpha_kernel(const InstState* in, 
   const int i = blockIdx.x;
   const bool act = in[i].act_eval != 0;
   const long long b0 = inst_off[i], b1 = inst_off[i + 1];
-  InstState s;
-  if (threadIdx.x == 0) s = in[i];
+  __shared__ InstState s;
+  state_in(in + i, &s);
   const double dq = flat_sum_odd<SCAL_TH>(table + b0, act ? b1 - b0 : 0, red);
-  if (threadIdx.x != 0) return;
-  cg_alpha_step(s, dq);
-  out[i] = s;
+  state_out(&s, out + i, [&](InstState& st) { cg_alpha_step(st, dq); });
 }
 
 // U of one vertex block, with the instance's step a and buffer
