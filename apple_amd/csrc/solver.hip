@@ -639,8 +639,15 @@ struct apl_solver {
   uint32_t* own = nullptr;  // per slot: vertex and OWNER_BIT
   int32_t* iso = nullptr;  // vertices without tets, then their instances
   int n_iso = 0;
-  double* hq = nullptr;    // per element block: quadratic form of the direction
-  InstState* st = nullptr;  // states after the step length (n), then after the decision (n)
+  // PNCG: per element block the quadratic form of the direction, and the states
+  // after the step length (n), then after the decision (n); kept from one
+  // apl_pncg_advance to the next
+  double* hq = nullptr;
+  InstState* st = nullptr;
+  // the same of the CG (d.Hd; after the beta step, after the alpha step): its
+  // own, so that a CG between two steps of a PNCG run leaves the run as it is
+  double* cg_hq = nullptr;
+  InstState* cg_st = nullptr;
   hipStream_t cap = nullptr;
   hipGraphExec_t gexec = nullptr;
   hipGraph_t graph = nullptr;
@@ -686,7 +693,7 @@ template <class R>
 static SolveArgs<R> solve_args(apl_solver* s, bool cg) {
   apl_mesh* m = s->mesh;
   SolveArgs<R> S;
-  S.st = s->st;
+  S.st = cg ? s->cg_st : s->st;
   S.out = nullptr;
   S.table = nullptr;
   S.n_table = 0;
@@ -699,7 +706,7 @@ static SolveArgs<R> solve_args(apl_solver* s, bool cg) {
   S.own = s->own;
   S.iso = s->iso;
   S.iso_inst = s->iso + s->n_iso;
-  S.hq = s->hq;
+  S.hq = cg ? s->cg_hq : s->hq;
   S.n_iso = s->n_iso;
   S.filter = m->L.n_inst > 1 ? 1 : 0;
   return S;
@@ -900,10 +907,10 @@ static int pncg_begin_t(apl_solver* s, const void* mu, const void* lam, void* x,
   return 0;
 }
 
-// the instances' states on the host (waits for the stream)
-static int read_states(apl_solver* s, hipStream_t st) {
+// the instances' states after an iteration on the host (waits for the stream)
+static int read_states(apl_solver* s, const InstState* states, hipStream_t st) {
   const size_t n = (size_t)s->mesh->L.n_inst;
-  APL_CHECK_HIP(hipMemcpyAsync(s->host_st, s->st + n, n * sizeof(InstState), hipMemcpyDeviceToHost, st));
+  APL_CHECK_HIP(hipMemcpyAsync(s->host_st, states + n, n * sizeof(InstState), hipMemcpyDeviceToHost, st));
   APL_CHECK_HIP(hipStreamSynchronize(st));
   return 0;
 }
@@ -931,7 +938,7 @@ static int pncg_advance_t(apl_solver* s, long long max_iters, int steps, hipStre
   const int n = (int)m->L.n_inst;
   std::vector<int32_t> target;
   if (steps > 0) {
-    if (read_states(s, st)) return -1;
+    if (read_states(s, s->st, st)) return -1;
     for (int i = 0; i < n; ++i) target.push_back(s->host_st[i].n_steps + steps);
   }
   long long ran = 0;
@@ -949,7 +956,7 @@ static int pncg_advance_t(apl_solver* s, long long max_iters, int steps, hipStre
     }
     run.done += K;
     ran += K;
-    if (read_states(s, st)) return -1;
+    if (read_states(s, s->st, st)) return -1;
     bool running = false, pending = false;
     for (int i = 0; i < n; ++i) {
       const bool r = s->host_st[i].status == APL_RUNNING;
@@ -967,7 +974,7 @@ static int pncg_end_t(apl_solver* s, apl_pncg_stats* stats, hipStream_t st) {
   PncgRun& run = s->run->r;
   if (copy_iterate<R>(s, run.x, st)) return -1;
   if (stats != nullptr) {
-    if (read_states(s, st)) return -1;
+    if (read_states(s, s->st, st)) return -1;
     for (int i = 0; i < (int)s->mesh->L.n_inst; ++i) {
       const InstState& h = s->host_st[i];
       apl_pncg_stats& o = stats[i];
@@ -1020,9 +1027,9 @@ static CgArgs<R> cg_args(apl_solver* s, const void* rhs, void* y, const uint8_t*
   A.nblocks = (int)m->L.nblocks;
   A.vblk_dots = m->d.vblk_dots;
   A.t_dots = m->d.vblk_dots + 2 * (size_t)A.nvblk;
-  A.in = s->st + m->L.n_inst;
+  A.in = s->cg_st + m->L.n_inst;
   A.out = nullptr;
-  A.hq = s->hq;
+  A.hq = s->cg_hq;
   A.V = (size_t)m->L.V;
   A.normal = 0;
   return A;
@@ -1034,7 +1041,7 @@ static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const vo
   apl_mesh* m = s->mesh;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   const unsigned ni = (unsigned)m->L.n_inst;
-  InstState *sa = s->st, *sb = s->st + ni;  // after the beta step, after the alpha step
+  InstState *sa = s->cg_st, *sb = s->cg_st + ni;  // after the beta step, after the alpha step
   const bool single = ni == 1 && m->L.nblocks > 0;
   SolveArgs<R> S = solve_args<R>(s, true);
   S.prm.rtol = rtol;
@@ -1062,7 +1069,7 @@ static int cg_iteration(apl_solver* s, const void* mu, const void* lam, const vo
     A.in = sa, A.out = sb;
     if (nvb) hipLaunchKernelGGL((cg_update_kernel<R, U_FUSED>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
   } else {
-    hipLaunchKernelGGL(cg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sa, sb, A.normal ? A.t_dots : s->hq,
+    hipLaunchKernelGGL(cg_alpha_kernel, dim3(ni), dim3(SCAL_TH), 0, st, sa, sb, A.normal ? A.t_dots : s->cg_hq,
                        A.normal ? m->d.inst_vblk_off : m->d.inst_blk_off);
     A.in = sb;
     if (nvb && ni == 1)
@@ -1082,7 +1089,7 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   const int n = (int)m->L.n_inst;
   const unsigned nvb = (unsigned)m->L.vblk_inst.size();
   CgArgs<R> A = cg_args<R>(s, rhs, y, mask);
-  hipLaunchKernelGGL(solve_init_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, st, s->st, n);
+  hipLaunchKernelGGL(solve_init_kernel, dim3((2 * n + 255) / 256), dim3(256), 0, st, s->cg_st, n);
   if (normal) {
     // the normal equations' right-hand side H b (b with fixed DOFs zeroed),
     // kept by the solver; the CG then runs on it
@@ -1100,7 +1107,7 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   if (fill<R>(A.hd, 3 * (long long)m->L.V, R(0), st)) return -1;
   if (launch_elem(m, s->material, W_H, mu, lam, x, nullptr, nullptr, A.hd, 0, st)) return -1;
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_DIAG>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
-  InstState* sb = s->st + n;
+  InstState* sb = s->cg_st + n;
   hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, sb, 0, m->d.vblk_dots, m->d.inst_vblk_off);
   if (nvb) hipLaunchKernelGGL((cg_vec_kernel<R, CG_PRECOND>), dim3(vec_grid(m)), dim3(NTH), 0, st, A);
   hipLaunchKernelGGL(cg_scalar_kernel, dim3(n), dim3(SCAL_TH), 0, st, sb, 1, m->d.vblk_dots, m->d.inst_vblk_off);
@@ -1154,7 +1161,7 @@ static int cg_solve_t(apl_solver* s, const void* mu, const void* lam, const void
   while (true) {
     APL_CHECK_HIP(hipGraphLaunch(s->cg_gexec, st));
     done += K;
-    if (read_states(s, st)) return -1;
+    if (read_states(s, s->cg_st, st)) return -1;
     bool running = false;
     for (int i = 0; i < n; ++i) running = running || s->host_st[i].status == APL_RUNNING;
     if (!running || done > (long long)max_iters + K) break;
@@ -1210,11 +1217,12 @@ int apl_solver_create(apl_mesh* m, int material, apl_solver** out) {
     total += (bytes + 255) / 256 * 256;
     return off;
   };
-  const size_t o_st = part(2 * (size_t)n * sizeof(InstState)), o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)),
-               o_p = part(2 * nv * 4 * rs), o_g = part(3 * nv * 4 * rs), o_cg = part(3 * nv * 4 * rs),
+  const size_t o_st = part(2 * (size_t)n * sizeof(InstState)), o_cg_st = part(2 * (size_t)n * sizeof(InstState)),
+               o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)), o_p = part(2 * nv * 4 * rs), o_g = part(3 * nv * 4 * rs), o_cg = part(3 * nv * 4 * rs),
                o_vecs = part(N_VECS * nv * 3 * rs),
                o_own = part((size_t)std::max<int64_t>(m->L.n_slots, 1) * sizeof(uint32_t)),
-               o_hq = part((size_t)std::max<int64_t>(m->L.nblocks, 1) * sizeof(double));
+               o_hq = part((size_t)std::max<int64_t>(m->L.nblocks, 1) * sizeof(double)),
+               o_cg_hq = part((size_t)std::max<int64_t>(m->L.nblocks, 1) * sizeof(double));
   auto fail = [&](const char* what) {
     set_error(what);
     (void)hipGetLastError();
@@ -1234,6 +1242,8 @@ int apl_solver_create(apl_mesh* m, int material, apl_solver** out) {
   s->vecs = base + o_vecs;
   s->own = (uint32_t*)(base + o_own);
   s->hq = (double*)(base + o_hq);
+  s->cg_st = (InstState*)(base + o_cg_st);
+  s->cg_hq = (double*)(base + o_cg_hq);
   // zeroed once: a solve overwrites what it reads
   if (hipMemset(s->mem, 0, o_own) != hipSuccess) return fail("hipMemset failed creating the solver");
   // owner slots, and the vertices that no tet touches
@@ -1329,7 +1339,7 @@ int apl_pncg_advance(apl_solver* s, int32_t steps, int64_t max_iters, void* x_ou
   if (x_out != nullptr && nx > 0 && (f32 ? copy_iterate<float>(s, x_out, st) : copy_iterate<double>(s, x_out, st)))
     return -1;
   if (state != nullptr) {
-    if (read_states(s, st)) return -1;
+    if (read_states(s, s->st, st)) return -1;
     for (int i = 0; i < (int)m->L.n_inst; ++i) {
       const InstState& h = s->host_st[i];
       apl_pncg_state& o = state[i];

@@ -303,7 +303,9 @@ int apl_pncg_solve(apl_solver* solver, const void* mu, const void* lam, void* x,
  * nullable) receives the current iterate and state (host, n_inst, nullable)
  * the per-instance optimizer state (the reference's opt_state fields);
  * apl_pncg_end writes the iterate into the x given to apl_pncg_begin and
- * fills stats.  apl_pncg_solve is begin + advance to the end + end. */
+ * fills stats.  apl_pncg_solve is begin + advance to the end + end.  Element
+ * passes on the mesh and apl_cg_solve of the same solver may run between two
+ * of these calls; apl_pncg_solve and apl_pncg_begin start anew. */
 typedef struct {
   int32_t status, n_steps, n_evals;
   int32_t ls_steps; /* line_search_state.step: backtracks of the last accepted step */
