@@ -742,7 +742,10 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
       for (int k = 0; k < SPT; ++k)
 #pragma unroll
         for (int ch = 0; ch < NCHA; ++ch) acc[k][ch] = R(0);
-      R e_acc = R(0), q_acc = R(0);
+      R e_acc = R(0);
+      // (v.Hv of the CG comes in FP64 and is added up in it: the step length
+      // hangs on it, and the unclamped forms of the tets cancel)
+      std::conditional_t<(WHAT & W_VQ) != 0, double, R> q_acc = 0;
       // one FP64 partial per wave and column into LDS, added in a fixed order
       // by one thread after the next barrier
       auto wave_partials = [&]() {

@@ -354,8 +354,9 @@ __global__ __launch_bounds__(SCAL_TH) void pncg_alpha_kernel(const InstState* in
 //      H d into the slot partials, and d.Hd per block
 //   U  vertex pass: the step from d.Hd (cg_alpha_step), q = H d summed from
 //      the partials, y += a d, r -= a q, z = r / diag, the dots r.r and r.z
-// d.Hd is summed per tet (FP64 over the tets) rather than from q, which would
-// need a vertex pass and a launch of its own between H and U.  An iteration of
+// d.Hd is summed over the tets (products and sums in FP64, as over the DOFs)
+// rather than from q, which would need a vertex pass and a launch of its own
+// between H and U.  An iteration of
 // a 32^3 cube takes 15.8 us (H 9.6, U 5.6; launches 1.6 us each), in five
 // launches it took 28.
 
@@ -1218,7 +1219,8 @@ int apl_solver_create(apl_mesh* m, int material, apl_solver** out) {
     return off;
   };
   const size_t o_st = part(2 * (size_t)n * sizeof(InstState)), o_cg_st = part(2 * (size_t)n * sizeof(InstState)),
-               o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)), o_p = part(2 * nv * 4 * rs), o_g = part(3 * nv * 4 * rs), o_cg = part(3 * nv * 4 * rs),
+               o_iso = part(sizeof(int)), o_x = part(2 * nv * 4 * sizeof(double)), o_p = part(2 * nv * 4 * rs),
+               o_g = part(3 * nv * 4 * rs), o_cg = part(3 * nv * 4 * rs),
                o_vecs = part(N_VECS * nv * 3 * rs),
                o_own = part((size_t)std::max<int64_t>(m->L.n_slots, 1) * sizeof(uint32_t)),
                o_hq = part((size_t)std::max<int64_t>(m->L.nblocks, 1) * sizeof(double)),

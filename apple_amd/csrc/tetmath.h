@@ -101,6 +101,15 @@ __host__ __device__ inline R ddot(const M3<R>& A, const M3<R>& B) {
   return s;
 }
 template <class R>
+__host__ __device__ inline double ddot_f64(const M3<R>& A, const M3<R>& B) {
+  double s = 0;
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) s += (double)A.m[i][j] * (double)B.m[i][j];
+  return s;
+}
+template <class R>
 __host__ __device__ inline R det3(const M3<R>& A) {
   return A.m[0][0] * (A.m[1][1] * A.m[2][2] - A.m[1][2] * A.m[2][1]) -
          A.m[0][1] * (A.m[1][0] * A.m[2][2] - A.m[1][2] * A.m[2][0]) +
@@ -804,7 +813,7 @@ struct TetOut {
   V3<R> h[4];   // max(dV diag H, 0)
   V3<R> hp[4];  // dV H v
   R hq;         // max(dV v^T H v, 0)
-  R vq;         // dV v^T H v
+  double vq;    // dV v^T H v, its products and sums in FP64 (the CG divides by their total)
   R dmu, dlam;  // dV (dP/dmu):dF(v), dV (dP/dlam):dF(v)
   R dact[6];    // dV d(P:dF(v))/da_k (muscle)
 };
@@ -904,7 +913,7 @@ __host__ __device__ inline void tet_eval(const TetGeom<R>& g0, R mu, R lam, cons
 #pragma unroll
             for (int j = 0; j < 3; ++j) Tm.m[i][j] = lc * C.m[i][j] + muV * dF.m[i][j] + sV * Hs.m[i][j];
           if constexpr ((WHAT & W_HP) != 0) corner_products(Tm, g, o.hp);
-          if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot(Tm, dF);
+          if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot_f64(Tm, dF);
         }
         if constexpr ((WHAT & W_MIX) != 0) {
           const M3<R> D = F_minus_cofF(G, I.trG);
@@ -983,7 +992,7 @@ __host__ __device__ inline void tet_eval(const TetGeom<R>& g0, R mu, R lam, cons
 #pragma unroll
           for (int j = 0; j < 3; ++j) T.m[i][j] = muV * (dF.m[i][j] - Qc.m[i][j]);
         corner_products(T, g, o.hp);
-        if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot(T, dF);
+        if constexpr ((WHAT & W_VQ) != 0) o.vq = ddot_f64(T, dF);
       }
       if constexpr ((WHAT & W_MIX) != 0) {
         o.dmu = g.dV * (S.sm1[0] * dM[0] + S.sm1[1] * dM[1] + S.sm1[2] * dM[2]);
