@@ -286,14 +286,12 @@ __host__ __device__ inline float fast_rsq(float x) {
 #endif
 }
 
-// 1/x, 1/sqrt(x), sqrt(x): the hardware approximations (about 1 ulp) in FP32,
+// 1/x and 1/sqrt(x): the hardware approximations (about 1 ulp) in FP32,
 // correctly rounded division and square root in FP64
 __host__ __device__ inline float recip(float x) { return fast_rcp(x); }
 __host__ __device__ inline double recip(double x) { return 1.0 / x; }
 __host__ __device__ inline float rsqrt_r(float x) { return fast_rsq(x); }
 __host__ __device__ inline double rsqrt_r(double x) { return 1.0 / sqrt(x); }
-__host__ __device__ inline float sqrt_r(float x) { return fast_sqrt(x); }
-__host__ __device__ inline double sqrt_r(double x) { return sqrt(x); }
 
 __host__ __device__ inline void jacobi_rotate_fast(float (&a)[3][3], M3<float>& V, int p, int q) {
   const float apq = a[p][q];
@@ -339,7 +337,7 @@ __host__ __device__ inline void swap_cols(M3<R>& V, R (&e)[3], int i, int j) {
 template <class R>
 __host__ __device__ inline void sigma_from(R e, R q, R& s, R& sm1) {
   if (fabs(e) < R(0.25) && q > R(0)) {
-    sm1 = e * recip(R(1) + sqrt_r(R(1) + e));
+    sm1 = e * recip(R(1) + sqrt(R(1) + e));
     s = R(1) + sm1;
   } else {
     s = q;
