@@ -627,6 +627,11 @@ __host__ __device__ inline void jacobi_fast_sweeps(float (&a)[3][3], M3<float>& 
 __host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, float (&e)[3]) {
   const float q = (a[0][0] + a[1][1] + a[2][2]) * (1.0f / 3.0f);
   float b00 = a[0][0] - q, b11 = a[1][1] - q, b22 = a[2][2] - q;
+  // what rounding left of the trace: it is part of l's equation, and where an
+  // element is squeezed (a near -I) it is as large as a's rounding (without this
+  // the stress error doubled at singular values about 0.3)
+  const float left = (b00 + b11 + b22) * (1.0f / 3.0f);
+  b00 -= left, b11 -= left, b22 -= left;
   float b01 = a[0][1], b02 = a[0][2], b12 = a[1][2];
   // scaled by the largest entry first: no square over- or underflows
   const float m = fmaxf(fmaxf(fmaxf(fabsf(b00), fabsf(b11)), fmaxf(fabsf(b22), fabsf(b01))),
