@@ -685,17 +685,21 @@ __host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, f
   set_col(V, 2, v3(top ? v2.x : v.x, top ? v2.y : v.y, top ? v2.z : v.z));
 }
 
-// The ARAP kernels' SVD: F^T F - I formed in FP64, then elements with
-// det F > 1/64 and det F > |F|^3 / 362 (large rotations and large strains
-// included) finish in FP32 (closed-form eigenvectors, QR), the inverted and
-// nearly flat ones in FP64 from the FP32 Jacobi basis (svd_finish_f64): there
-// the rotation-variant sign convention hinges on the sign of det F and on
-// comparisons of nearly equal |sigma| that FP32 can get the other way, and
-// the Jacobi basis keeps an already diagonal F^T F as it is, ties included.
-// The first threshold keeps the FP32 det3's rounding (~1e-7 |F|^3) far from
-// deciding the branch; the second is met by elements drawn out more than
-// about 10:1, where the rotation about the long axis amplifies FP32 rounding
-// by sigma_0 / (sigma_1 + sigma_2).  Only those elements' branch is divergent.
+// The ARAP kernels' SVD: F^T F - I formed in FP64, then by shape:
+//  * det F > |F|^3 / 10 and det F > 1/64: closed-form eigenvectors, FP32 QR
+//    (any rotation; elements drawn out to 2.6:1, flattened to 3.3:1, squeezed to
+//    a quarter of their size).
+//  * det F > |F|^3 / 362 and det F > 1/64: Jacobi sweeps, FP32 sort and QR.
+//    FP32 rounding is amplified by sigma_0^2 / (sigma_1 (sigma_1 + sigma_2)) in
+//    the rotation about an element's long axis; the closed form's rounding
+//    passes the sweeps' from 2.8:1 on (root mean square of the projected Hessian's
+//    error at 4:1 1.6e-7 against 1.4e-7, at 8:1 4.7e-7 against 2.9e-7).
+//  * inverted, nearly flat and further drawn-out elements (19:1): FP64 from the
+//    Jacobi basis (svd_finish_f64).  There the rotation-variant sign convention
+//    hinges on the sign of det F and on comparisons of nearly equal |sigma| that
+//    FP32 can get the other way, and the Jacobi basis keeps an already diagonal
+//    F^T F as it is, ties included.  1/64 keeps the FP32 det3's rounding
+//    (~1e-7 |F|^3) far from deciding the branch.
 __host__ __device__ inline Svd<float> svd_rv_fast(const M3<float>& G) {
   float a[3][3];
   ftf_minus_i_f64(G, a);
@@ -705,13 +709,16 @@ __host__ __device__ inline Svd<float> svd_rv_fast(const M3<float>& G) {
   F.m[1][1] += 1.0f;
   F.m[2][2] += 1.0f;
   const float det = det3(F), f2 = 3.0f + (a[0][0] + a[1][1] + a[2][2]);
-  if (det > 0.015625f && det * det * 131072.0f > f2 * f2 * f2) {
-    float e[3];
+  const float d2 = det > 0.015625f ? det * det : 0.0f, f6 = f2 * f2 * f2;
+  float e[3];
+  if (d2 * 100.0f > f6) {
     eig_sym3(a, V, e);
-    return qr_sigma(G, V, e);
+  } else {
+    jacobi_fast_sweeps(a, V);
+    if (!(d2 * 131072.0f > f6)) return svd_finish_f64(G, V);
+    sort_eig(a, V, e);
   }
-  jacobi_fast_sweeps(a, V);
-  return svd_finish_f64(G, V);
+  return qr_sigma(G, V, e);
 }
 
 template <class R>
