@@ -685,6 +685,17 @@ __host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, f
   set_col(V, 2, v3(top ? v2.x : v.x, top ? v2.y : v.y, top ? v2.z : v.z));
 }
 
+// Whether p holds in every active lane of the wave (on the host: of the one element)
+__host__ __device__ inline bool wave_all(bool p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  int all = __builtin_amdgcn_ballot_w64(!p) == 0ull;
+  asm("" : "+v"(all));  // a lane's own value for the compiler: a uniform branch here costs 6 VGPRs, H v a wave per SIMD
+  return all != 0;
+#else
+  return p;
+#endif
+}
+
 // The ARAP kernels' SVD: F^T F - I formed in FP64, then by shape:
 //  * det F > |F|^3 / 10 and det F > 1/64: closed-form eigenvectors, FP32 QR
 //    (any rotation; elements drawn out to 2.6:1, flattened to 3.3:1, squeezed to
@@ -700,6 +711,11 @@ __host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, f
 //    FP32 can get the other way, and the Jacobi basis keeps an already diagonal
 //    F^T F as it is, ties included.  1/64 keeps the FP32 det3's rounding
 //    (~1e-7 |F|^3) far from deciding the branch.
+// The closed form is taken by whole waves: one whose tets do not all allow it
+// takes the sweeps for all of them.  With both in one wave, meshes full of
+// inverted tets were slower than by sweeps alone (64^3, 33 % inverted: 83.1 us
+// for the E, g, diag H pass, now 78.7, by sweeps alone 80.2; none inverted 45.4,
+// by sweeps alone 55.9).
 __host__ __device__ inline Svd<float> svd_rv_fast(const M3<float>& G) {
   float a[3][3];
   ftf_minus_i_f64(G, a);
@@ -711,7 +727,7 @@ __host__ __device__ inline Svd<float> svd_rv_fast(const M3<float>& G) {
   const float det = det3(F), f2 = 3.0f + (a[0][0] + a[1][1] + a[2][2]);
   const float d2 = det > 0.015625f ? det * det : 0.0f, f6 = f2 * f2 * f2;
   float e[3];
-  if (d2 * 100.0f > f6) {
+  if (wave_all(d2 * 100.0f > f6)) {
     eig_sym3(a, V, e);
   } else {
     jacobi_fast_sweeps(a, V);
