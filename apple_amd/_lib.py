@@ -193,19 +193,25 @@ _calls = None
 
 def calls():
     """The extension module that calls the library from torch tensors
-    (csrc/python/tensor_calls.cpp) and the entries it calls, loaded once
-    (raises if it has not been built): (module, apl_elem_eval,
-    apl_elem_mixed_activation, apl_mesh_set_activation)."""
+    (csrc/python/tensor_calls.cpp) and the entries it calls, loaded once:
+    (module, apl_elem_eval, apl_elem_mixed_activation,
+    apl_mesh_set_activation).  Empty, after a warning, where the module has
+    not been built: the callers then check their arguments in Python, which
+    takes 7 us more per call."""
     global _calls
     if _calls is None:
         import importlib.util
+        import warnings
 
         import torch  # noqa: F401  (the module is linked against its libraries)
 
-        L = lib()
         path = os.path.join(os.path.dirname(LIB_PATH), "tensor_calls.so")
         if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: build it with `python -m apple_amd.build`")
+            _calls = ()
+            warnings.warn(f"{path} is missing (build it with `python -m apple_amd.build`): element calls check "
+                          "their arguments in Python", RuntimeWarning, stacklevel=2)
+            return _calls
+        L = lib()
         with _lock:
             if _calls is None:
                 spec = importlib.util.spec_from_file_location("tensor_calls", path)

@@ -164,12 +164,14 @@ class DeviceMesh:
     def set_activation(self, activation: torch.Tensor | None) -> None:
         """Bind the (T, 6) activation that muscle-law launches read (the mesh
         keeps the pointer; this object keeps the tensor alive)."""
-        mod, _, _, entry = _lib.calls()
-        rc = mod.set_activation(entry, self._handle.value, 0, self._spec, activation)
-        if rc is not None:
-            _lib.check(rc)
-            self._activation = activation
-            return
+        native = _lib.calls()
+        if native:
+            mod, _, _, entry = native
+            rc = mod.set_activation(entry, self._handle.value, 0, self._spec, activation)
+            if rc is not None:
+                _lib.check(rc)
+                self._activation = activation
+                return
         if activation is not None:
             ptr(activation, dtype=self.dtype, device=self.device, shape=(self.n_tets, 6), name="activation")
         _lib.check(_lib.lib().apl_mesh_set_activation(self._handle, activation.data_ptr() if activation is not None else None))
@@ -253,14 +255,17 @@ class DeviceMesh:
         accumulate=False,
     ) -> None:
         """One fused element pass writing (or adding into) the given outputs."""
-        mod, entry, _, _ = _lib.calls()
-        rc = mod.elem_eval(entry, self._handle.value, _raw_stream(self.device.index), self._spec, material, accumulate,
-                           mu, lam if material != _lib.APL_ARAP else None, u, p, energy, grad, hess_diag, hess_prod,
-                           hess_quad, dmu, dlam)
-        if rc is not None:
-            _lib.check(rc)
-            return
-        # an argument is not a plain tensor of the form it has to have: say which, or take it as it is
+        native = _lib.calls()
+        if native:
+            mod, entry, _, _ = native
+            rc = mod.elem_eval(entry, self._handle.value, _raw_stream(self.device.index), self._spec, material,
+                               accumulate, mu, lam if material != _lib.APL_ARAP else None, u, p, energy, grad,
+                               hess_diag, hess_prod, hess_quad, dmu, dlam)
+            if rc is not None:
+                _lib.check(rc)
+                return
+        # no module, or an argument is not a plain tensor of the form it has to have: say which,
+        # or take it as it is
         what = 0
         if energy is not None:
             what |= _lib.APL_ENERGY
@@ -301,12 +306,14 @@ class DeviceMesh:
     def mixed_activation(self, mu, lam, u, p, dact, *, dmu=None, dlam=None, accumulate=False) -> None:
         """Muscle law: per-tet p^T d(grad)/d(activation) into dact (T, 6), and
         optionally p^T d(grad)/d(mu), d/d(lambda) in the same pass."""
-        mod, _, entry, _ = _lib.calls()
-        rc = mod.elem_mixed_activation(entry, self._handle.value, _raw_stream(self.device.index), self._spec,
-                                       accumulate, mu, lam, u, p, dact, dmu, dlam)
-        if rc is not None:
-            _lib.check(rc)
-            return
+        native = _lib.calls()
+        if native:
+            mod, _, entry, _ = native
+            rc = mod.elem_mixed_activation(entry, self._handle.value, _raw_stream(self.device.index), self._spec,
+                                           accumulate, mu, lam, u, p, dact, dmu, dlam)
+            if rc is not None:
+                _lib.check(rc)
+                return
         tet = dict(dtype=self.dtype, device=self.device, shape=(self.n_tets,))
         _lib.check(
             _lib.lib().apl_elem_mixed_activation(

@@ -1,0 +1,44 @@
+"""The extension module that calls the library from torch tensors is an
+accelerator: without it the library builds and every call takes the checked
+Python path, as it did before there was one."""
+
+import warnings
+
+import numpy as np
+import pytest
+import torch
+
+from apple_amd import _lib, fem
+from apple_amd.mesh import Region, cube
+
+
+def test_a_library_without_the_module_is_used_as_it_is(tmp_path, monkeypatch):
+    monkeypatch.setattr(_lib, "LIB_PATH", str(tmp_path / "libapple_amd.so"))
+    monkeypatch.setattr(_lib, "_calls", None)
+    with pytest.warns(RuntimeWarning, match="tensor_calls.so is missing"):
+        assert not _lib.calls()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert not _lib.calls()  # said once
+
+
+@pytest.mark.gpu
+def test_calls_without_the_module_give_the_same(monkeypatch):
+    m = cube(3)
+    rng = np.random.default_rng(0)
+    m.cell_data["mu"] = 1e4 * np.exp(0.5 * rng.standard_normal(m.n_cells))
+    m.cell_data["lambda"] = 10 * m.cell_data["mu"]
+    m.cell_data["activation"] = 0.1 * rng.standard_normal((m.n_cells, 6))
+    pot = fem.StableNeoHookeanMuscle.from_region(Region.from_mesh(m), device="cuda")
+    t = lambda a: torch.as_tensor(a, dtype=torch.float32, device="cuda")  # noqa: E731
+    u, p = t(0.01 * rng.standard_normal(m.points.shape)), t(rng.standard_normal(m.points.shape))
+
+    def calls():
+        g, e = torch.zeros_like(u), torch.zeros(1, dtype=torch.float64, device="cuda")
+        pot.fused(u, e, g, None)
+        return [g, e, *pot.mixed_derivative_prod(u, p).values()]
+
+    native = calls()
+    monkeypatch.setattr(_lib, "_calls", ())
+    for a, b in zip(native, calls()):
+        assert torch.equal(a, b) and a.abs().max() > 0
