@@ -57,9 +57,10 @@ def current_stream(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-# The same for a device whose index is known and that is in use already
-# (no Stream object: 0.1 us instead of 1.9)
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# The same for a device whose index is known and that is in use already (no
+# Stream object: 0.1 us instead of 1.9; a PyTorch without devices has no such lookup)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 class DeviceMesh:

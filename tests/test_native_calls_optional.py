@@ -2,6 +2,9 @@
 accelerator: without it the library builds and every call takes the checked
 Python path, as it did before there was one."""
 
+import os
+import subprocess
+import sys
 import warnings
 
 import numpy as np
@@ -10,6 +13,8 @@ import torch
 
 from apple_amd import _lib, fem
 from apple_amd.mesh import Region, cube
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def test_a_library_without_the_module_is_used_as_it_is(tmp_path, monkeypatch):
@@ -42,3 +47,14 @@ def test_calls_without_the_module_give_the_same(monkeypatch):
     monkeypatch.setattr(_lib, "_calls", ())
     for a, b in zip(native, calls()):
         assert torch.equal(a, b) and a.abs().max() > 0
+
+
+def test_import_without_the_raw_stream_lookup():
+    """A PyTorch without CUDA or ROCm has no torch._C._cuda_getCurrentRawStream: the package imports there."""
+    code = ("import torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'):\n"
+            "    del torch._C._cuda_getCurrentRawStream\n"
+            "import apple_amd.runtime, apple_amd.fem, apple_amd.mesh\n"
+            "print('imported')\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=ROOT)
+    assert r.returncode == 0 and r.stdout.strip().endswith("imported"), r.stderr
