@@ -74,22 +74,26 @@ def _build_module() -> None:
 
 
 def build(verbose: bool = True) -> str:
-    """Compile every source and link the shared library and the extension
-    module; returns the library's path."""
+    """Compile every source and link the shared library, then the extension
+    module (left out where there is no PyTorch: the C ABI needs none);
+    returns the library's path."""
     os.makedirs(OBJDIR, exist_ok=True)
     srcs = sources()
     jobs = min(len(srcs) + 1, max(1, min(16, os.cpu_count() or 1)))
     with concurrent.futures.ThreadPoolExecutor(jobs) as ex:
         module = ex.submit(_build_module)
         objs = list(ex.map(_compile, srcs))
-        module.result()
-    out = os.path.join(LIBDIR, LIBNAME)
-    tmp = out + ".tmp"
-    cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"link failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
-    os.replace(tmp, out)
+        out = os.path.join(LIBDIR, LIBNAME)
+        tmp = out + ".tmp"
+        cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"link failed: {' '.join(cmd)}\n{proc.stdout}\n{proc.stderr}")
+        os.replace(tmp, out)
+        try:
+            module.result()
+        except ImportError as e:
+            print(f"{MODULE}.so not built: {e}", file=sys.stderr)
     if verbose:
         print(f"built {out}", file=sys.stderr)
     return out

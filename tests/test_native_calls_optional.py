@@ -2,6 +2,7 @@
 accelerator: without it the library builds and every call takes the checked
 Python path, as it did before there was one."""
 
+import ctypes
 import os
 import subprocess
 import sys
@@ -11,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from apple_amd import _lib, fem
+from apple_amd import _lib, build, fem
 from apple_amd.mesh import Region, cube
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -58,3 +59,28 @@ def test_import_without_the_raw_stream_lookup():
             "print('imported')\n")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, cwd=ROOT)
     assert r.returncode == 0 and r.stdout.strip().endswith("imported"), r.stderr
+
+
+def test_the_library_is_linked_whatever_becomes_of_the_module(tmp_path, monkeypatch):
+    """The C ABI needs neither PyTorch's nor Python's headers."""
+    src = tmp_path / "one.cpp"
+    src.write_text('extern "C" int one() { return 1; }\n')
+    monkeypatch.setattr(build, "LIBDIR", str(tmp_path / "lib"))
+    monkeypatch.setattr(build, "OBJDIR", str(tmp_path / "lib" / "obj"))
+    monkeypatch.setattr(build, "sources", lambda: [str(src)])
+    lib = tmp_path / "lib" / build.LIBNAME
+
+    def fails():
+        raise RuntimeError("compile failed: no headers")
+
+    monkeypatch.setattr(build, "_build_module", fails)
+    with pytest.raises(RuntimeError, match="no headers"):  # said, and the library is there
+        build.build(verbose=False)
+    assert ctypes.CDLL(str(lib)).one() == 1
+    lib.unlink()
+
+    def no_torch():
+        raise ImportError("no module named torch")
+
+    monkeypatch.setattr(build, "_build_module", no_torch)
+    assert build.build(verbose=False) == str(lib) and lib.exists()
