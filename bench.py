@@ -12,7 +12,7 @@ restatement of the reference's separate fun/grad/hess_diag passes, timed on
 the host), PNCG solves/s at 1e-6 relative gradient norm, the ARAP pass, and a
 batched-vs-plain solve comparison.
 
-Usage: python bench.py [--steps K] [--warmup W] [--gpus 1] [--quick]
+Usage: python bench.py [--steps K] [--warmup W] [--gpus 1] [--quick] [--details FILE]
 """
 
 from __future__ import annotations
@@ -35,6 +35,22 @@ HBM_PEAK_GBS = 8000.0
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+def contract_line(out: dict) -> str:
+    """The result as one JSON line of under 10,000 characters (with every
+    instance of the combined case it was 27,000, and readers that keep the end
+    of a run's output lost its head): nested numbers to six digits, without the
+    per-instance entries, which --combined-only and --details give."""
+
+    def short(v):
+        if isinstance(v, dict):
+            return {k: short(w) for k, w in v.items() if k != "per_instance"}
+        if isinstance(v, list):
+            return [short(w) for w in v]
+        return float(f"{v:.6g}") if isinstance(v, float) else v
+
+    return json.dumps({k: short(v) if isinstance(v, dict) else v for k, v in out.items()})
 
 
 def make_cube_problem(n, material, dtype, device, seed_mu=1, seed_noise=0, noise_frac=0.1, chunks=1, seed_act=8):
@@ -280,6 +296,7 @@ def main():
     ap.add_argument("--batched-meshes", type=int, default=256)
     ap.add_argument("--cpu-threads", type=int, default=0,
                     help="threads of the multi-threaded CPU baseline (0: every core available to the process)")
+    ap.add_argument("--details", metavar="FILE", help="also write the whole result (every instance, all digits) there")
     ap.add_argument("--profile-pass", action="store_true",
                     help="only run pass-A launches and a reference copy (for rocprofv3 counter runs)")
     ap.add_argument("--profile-hess-prod", action="store_true",
@@ -548,7 +565,10 @@ def main():
         log(f"[bench] CPU baseline (C restatement, {args.cpu_threads} threads and 1 thread, {host_cpu()})")
         out["cpu_baseline"] = cpu_baseline(prob, target_s=12.0, threads=args.cpu_threads)
         out["cpu_baseline_1thread"] = cpu_baseline(prob, target_s=12.0, threads=1)
-    print(json.dumps(out), flush=True)
+    if args.details:
+        with open(args.details, "w") as fh:
+            json.dump(out, fh, indent=1)
+    print(contract_line(out), flush=True)
 
 
 def make_cube_instances(n_meshes, lo, hi, seed_sizes, seed_mat, noise_frac=0.1):
