@@ -35,10 +35,12 @@ struct FinishArgs {
 
 // The vertex sums wait for one chain, offsets -> partials -> sums.  FP32
 // passes of six channels on meshes of up to two vertex blocks per CU have all
-// of a thread's loads of the partials in flight at once (WINDOW: 45^3 5.3 ->
-// 4.3 us); with more blocks resident (64^3), three channels or FP64 the loop
-// of four is 0.2-0.4 us faster.  With one instance (SINGLE) the block's
-// vertices follow from its number.
+// of a thread's loads of the partials in flight at once (WINDOW).  Whole SNH
+// evaluations, us, with the loop of four / with the window: 141 vertex blocks
+// 12.3 / 11.3, 381 19.2 / 18.3, 489 20.9 / 20.1, 519 21.3 / 20.8, 724 24.9 / 24.5,
+// 887 28.5 / 28.5, 1,073 32.0-32.3 / 32.3; with three channels or in FP64 the
+// loop is 0.2-0.4 us faster.  With one instance (SINGLE) the block's vertices
+// follow from its number.
 template <class R, int NCH, bool SINGLE, bool WINDOW>
 __global__ __launch_bounds__(NTH) void finish_kernel(FinishArgs<R> A) {
   __shared__ double eq[2 * (NTH / 64 + 1)];

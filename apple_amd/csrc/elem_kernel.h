@@ -21,8 +21,9 @@
 //    vertex-major buffer (a vertex's partials contiguous, in block order);
 //    the vertex pass adds each vertex's contiguous run;
 //  * energies and quadratic forms are summed per thread, then in FP64 by a
-//    fixed wave-shuffle tree into one partial per wave (no block barrier),
-//    and a per-instance pass adds the wave partials in a fixed order;
+//    fixed DPP tree per wave and over the block's four waves in order (behind
+//    the barrier of the slot sums where a pass has them); a per-instance pass
+//    adds the blocks' values in a fixed order;
 //  * the grid is persistent and XCD-aware: workgroup i runs on XCD i % 8, and
 //    XCD x walks every eighth chunk of up to 16 consecutive blocks, so
 //    neighbouring blocks (which share vertices) mostly hit the same L2 while
@@ -70,7 +71,6 @@ struct ElemArgs {
   int T;
   int nblocks;  // blocks this launch visits (the list's length with a list)
   int nloc_max;
-  int chunks;
   int accumulate;
 };
 
@@ -78,10 +78,6 @@ struct ElemArgs {
 template <class T>
 struct alignas(4 * sizeof(T)) Vec4 {
   T v[4];
-};
-template <class T>
-struct alignas(2 * sizeof(T)) Vec2 {
-  T v[2];
 };
 
 // The solver's element passes.  WHAT carries one of these staging modes
@@ -571,8 +567,8 @@ __device__ __forceinline__ void elem_body(const ElemArgs<R, X>& A, const SOLVE& 
   // Passes without a scatter phase have registers to spare: each thread
   // loads the next block's staging inputs (its slot tid) while the current
   // block finishes, so that block's staging waits on no global load.  Not in
-  // the scatter passes nor with FP64 displacements: there the registers
-  // cost a wave per SIMD and the gain disappears (measured).
+  // the scatter passes, where the registers cost a wave per SIMD and the gain
+  // disappears (measured), nor in the solver's, which stage other records.
   constexpr bool PREFETCH = !SCATTER && !SOLVER;
   int pf_b = -1;
   X pf_x[3] = {X(0), X(0), X(0)};
@@ -1036,7 +1032,6 @@ static ElemArgs<R, X> make_args(apl_mesh* m, const void* mu, const void* lam, co
   A.blk_list = nullptr;
   A.nblocks = (int)m->L.nblocks;
   A.nloc_max = m->L.nloc_max;
-  A.chunks = m->L.chunks;
   A.accumulate = accumulate;
   return A;
 }
@@ -1071,9 +1066,13 @@ inline int64_t launch_blocks(const apl_mesh* m, int mat) { return m->model ? m->
 // round of persistent workgroups, except for the VALU-heavy ARAP gradient
 // passes (4 waves per SIMD) and the Hessian-vector pass, which run faster
 // with a second, non-resident round that the hardware dispatches as
-// workgroups of the first finish (a dynamic balance of the last blocks;
-// measured on the 64^3 cube: ARAP pass A 58.6 -> 55.1 us, SNH H v 30.3 ->
-// 27.4 us, while SNH pass A and the quadratic-form passes are fastest at 100).
+// workgroups of the first finish (a dynamic balance of the last blocks).
+// Whole FP32 evaluations, us at 100 / 200: 64^3 ARAP E, g, diag H 49.2 / 45.6,
+// H v of SNH 28.0 / 27.7, muscle 33.0 / 30.1, ARAP 39.1 / 38.2; at 45^3 (1,780
+// blocks) all equal but ARAP's H v, 19.2 / 20.9.  The passes left at 100 gain
+// up to 5 % from 200 at 64^3 now that a block takes fewer latencies (SNH
+// E, g, diag H 33.1 / 31.8, muscle 38.6 / 36.8, v.Hv of SNH 22.2 / 21.8, ARAP
+// 31.1 / 30.0) and nothing to 32^3; the autotuner chooses per mesh.
 constexpr int default_grid_pct(int mat, unsigned what) {
   return ((what & W_HP) != 0 || (mat == MAT_ARAP && (what & (W_G | W_H)) != 0)) ? 200 : 100;
 }

@@ -34,12 +34,20 @@ constexpr int STATE_DOUBLES = sizeof(InstState) / 8;
 constexpr int SCAL_TH = 1024;
 
 // A single instance's scalar steps ride in the element pass that follows
-// them up to these table sizes (FUSE_BLOCKS element blocks for the step
-// length, FUSE_VBLOCKS vertex blocks of 16 columns for the decision): every
-// workgroup reads the whole table, so beyond them the launch saved costs
-// more in the L2 than it gives (64^3 cubes, 5,120 blocks: the trial pass grew
-// by 3.8 us, the launch is 4.7 us and the whole solve was slower).
-// FUSE_CG_VBLOCKS: the CG's two columns per vertex block, by the same measure.
+// them up to these table sizes: FUSE_BLOCKS element blocks for the step length
+// (and for d.Hd in the CG's update), FUSE_VBLOCKS vertex blocks of 16 columns for
+// the decision, FUSE_CG_VBLOCKS of two columns for the CG's beta.  Every
+// workgroup reads the whole table and the pass takes more registers, so the gain
+// falls with size.  Whole iterations of SNH in FP32, us, in the pass / as a launch:
+//   step length  20 blocks 19.7 / 21.3, 640 25.8 / 27.2, 2,028 42.1 / 44.0, 2,160
+//                45.1 / 46.9, 4,012 64.8 / 65.2 (about the end of the short tables)
+//   decision     6 vertex blocks 19.7 / 20.9, 141 25.8 / 26.9, 198 29.3 / 30.2
+//   CG's beta    6 13.0 / 14.2, 141 15.9 / 17.0, 270 20.5 / 22.2, 290 23.1 / 23.1,
+//                356 25.5 / 24.6, 844 37.8 / 37.1
+// The first two lines keep a margin to where the gain ends.  The CG's is generous:
+// from 290 vertex blocks on the launch is up to 5 % faster in FP32 (SNH FP64: the
+// pass, to 460), for ARAP from about 200, and for ARAP and muscle in FP64 from
+// about 100 (141: 25.8 / 23.2 and 24.6 / 22.2).
 constexpr int FUSE_BLOCKS = 2048, FUSE_VBLOCKS = 192, FUSE_CG_VBLOCKS = 1024;
 static_assert(FUSE_BLOCKS <= 4 * SCAL_TH && FUSE_VBLOCKS * N_DOTS <= 4 * SCAL_TH && FUSE_CG_VBLOCKS * 2 <= 4 * SCAL_TH,
               "short tables (flatsum.h)");
