@@ -621,9 +621,9 @@ __host__ __device__ inline void jacobi_fast_sweeps(float (&a)[3][3], M3<float>& 
 // those two are; the plane orthogonal to it (orthonormal basis after Duff et
 // al., "Building an Orthonormal Basis, Revisited", JCGT 2017) is left with a
 // 2x2 problem, one exact rotation.
-// Against four cyclic Jacobi sweeps the ARAP pass issues 979 instead of 1,350
-// VALU instructions per 64 tets; the 64^3 pass went from 64.4 to 53.9 us and
-// its error against 64 bits from 2.8e-7 to 2.3e-7.
+// Against four cyclic Jacobi sweeps the ARAP pass issues 1,062 instead of 1,350
+// VALU instructions per 64 tets; the element kernel takes 44.5 instead of 55.1 us
+// at 64^3 (VALU issue: 35 us), the error against 64 bits went from 2.9e-7 to 2.3e-7.
 __host__ __device__ inline void eig_sym3(const float (&a)[3][3], M3<float>& V, float (&e)[3]) {
   const float q = (a[0][0] + a[1][1] + a[2][2]) * (1.0f / 3.0f);
   float b00 = a[0][0] - q, b11 = a[1][1] - q, b22 = a[2][2] - q;
